@@ -348,6 +348,10 @@ int nslg_paged_decode_grouped_rope_append(
  *               the true max only costs that order, never correctness)
  *   out         [T] rows of Hq*D elements at stride out_stride
  *   sm_scale    positive and finite (EINVAL otherwise)
+ *   workspace   of nslg_paged_prefill_workspace_size bytes, not shared with a call
+ *               that may run at the same time: a call of few row tiles then cuts its
+ *               keys into runs and merges them (a second launch). Null or smaller:
+ *               fewer runs, or one and no use of the workspace
  * Supported: f16, bf16 with D in {64, 128, 256} (MFMA); f32 with D in {64, 128,
  * 256} (the VALU kernel of nslg_paged_decode's f32 path); 1 <= Hq/Hkv <= 16.
  */

@@ -26,6 +26,14 @@
 // The sequence's page ids for the workgroup's key range sit in LDS (windows of
 // 2048 pages), so tile loads never wait on index loads.
 //
+// A workgroup takes a CU, so a call of few row tiles (one request's chunk: 64 of the 256
+// CUs at 512 tokens, 8 at 16) is bound by how long one workgroup walks its keys. Given a
+// workspace, such a call cuts each tile's keys into runs, one workgroup each, whose fp32
+// rows prefill_merge_kernel combines. Measured (32/8 heads x 128, one sequence, both
+// launches): f16 512 tokens over 4096 keys 147 -> 61 us, over 16000 501 -> 157, 16 over
+// 2048 52.5 -> 19.3; bf16 512 over 6007 286 -> 91 us, and two of 512 over 2k at D = 256
+// 160 -> 107.
+//
 // Built with -fno-honor-nans (nanoslg_amd/_build.py): the running maxima are
 // taken with plain v_max/v_max3 instead of NaN-quieting ones.
 #include "nslg_common.h"
@@ -37,6 +45,9 @@ namespace {
 
 constexpr int kPageWin = 2048;                     // page ids per LDS window
 constexpr float kRescaleSlack = 8.0f;
+constexpr int kCUs = 256;       // compute units of the part
+constexpr int kMaxSplits = 32;  // runs of keys per row tile
+constexpr int kMinRun = 1;      // key tiles per run, at least (2: 16 tokens over 512 16.6 us, with 1 14.4)
 
 // Tile shape per head dim: column blocks of 16 query rows per wave, keys per LDS
 // tile, waves per workgroup. D = 64, 128: two column blocks per wave and 128-key
@@ -97,6 +108,15 @@ struct PrefillParams {
   int64_t v_new_stride;
   uint32_t k_new_bytes;  // bytes of k_new's rows (the grid's or total_q), < 4 GiB
   uint32_t v_new_bytes;
+  // Split keys (the kSplit kernel): workgroup (row tile, y of `splits`) takes a run of
+  // the tile's key tiles and leaves unnormalised rows for the merge. Row (token t, query
+  // head) of run y is row (y * total_q + t) * Hq + head of part_o / part_ml, and
+  // part_count holds the runs of each (token, head): 1 for a row already in `out`.
+  int32_t splits;
+  int64_t total_q;
+  float* part_o;        // [splits, total_q, Hq, D]
+  float2* part_ml;      // [splits, total_q, Hq]: running max (log2 units) and row sum
+  int32_t* part_count;  // [total_q, Hq]
 };
 
 // Word 3 of a raw (untyped, unswizzled) buffer resource on CDNA: 32-bit data format,
@@ -190,7 +210,7 @@ __device__ inline bool locate_tile(const PrefillParams& p, int g, int& b, int& t
   return false;
 }
 
-template <typename T, int D>
+template <typename T, int D, bool kSplit>
 __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_kernel(PrefillParams p) {
   constexpr int kCB = PrefillTile<D>::kCB;
   constexpr int kKeys = PrefillTile<D>::kKeys;
@@ -221,16 +241,22 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   // XCD-aware order: workgroup i runs on XCD i % 8, so work item
   // w = (i % 8) * per_xcd + i / 8 gives each XCD a contiguous run of row tiles of
   // one KV head, which read the same K/V and so share that XCD's L2.
-  const int w = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
+  // kSplit: work item = workgroup, the tiles' first slots before the last ones and the
+  // (KV head, run) pairs in turn: the empty slots of the grid's upper bound then come
+  // last. Between the full ones they keep CUs from work: a tile of 17 runs, every other
+  // slot empty, took 35 us, of 9 runs 13 us (16 of an XCD's CUs got the full slots).
+  const int w = kSplit ? (int)blockIdx.x : (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
   if (w >= p.num_work) {
     if (w < p.num_work + p.pad_work)
       zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, w - p.num_work, p.out, p.out_stride,
                     (int64_t)p.num_qo_heads * D, (int64_t)p.batch * p.grid_width);
     return;
   }
-  const int h = w / p.row_tiles;
+  const int runs = p.num_kv_heads * p.splits;
+  const int run = kSplit ? w % runs : w / p.row_tiles;  // (KV head, run of keys)
+  const int h = kSplit ? run / p.splits : run;
   int b = 0, tile = 0;
-  const int g = w - h * p.row_tiles;
+  const int g = kSplit ? w / runs : w - run * p.row_tiles;
   // longest-first rounds when the host's round count covers every sequence (it came
   // from the caller's max_q); otherwise the packed order, which the grid also fits
   const bool rounds = p.by_round > 0 && most_tiles(p) <= p.by_round;
@@ -249,7 +275,18 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   // keys this workgroup needs: up to the last row's position (inclusive)
   const int last_row = min(row0_wg + kRowsPerWG, nrows) - 1;
   const int kv_end = min(L, start + last_row / G + 1);
-  const int n_kt = (kv_end + kKeys - 1) / kKeys;
+  int kt_first = 0;
+  int n_kt = (kv_end + kKeys - 1) / kKeys;
+  int parts = 1;
+  if constexpr (kSplit) {
+    // equal runs of key tiles, of at least kMinRun tiles each
+    const int split = run - h * p.splits;
+    const int per = max((n_kt + p.splits - 1) / p.splits, kMinRun);
+    parts = max((n_kt + per - 1) / per, 1);
+    if (split >= parts) return;
+    kt_first = split * per;
+    n_kt = min(n_kt, kt_first + per);
+  }
   const int32_t* idx = p.indices + p.indptr[b];
   const int np_seq = p.indptr[b + 1] - p.indptr[b];
   const int ps = p.page_size;
@@ -602,17 +639,17 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
     }
   };
 
-  if (n_kt > 0) {
-    load_pages(0);
+  if (n_kt > kt_first) {
+    load_pages(kt_first * kKeys);
     __syncthreads();
-    fetch_half(0, 0);
-    stash_half(0, 0);
-    fetch_half(0, 1);
-    stash_half(0, 1);
+    fetch_half(kt_first, 0);
+    stash_half(kt_first & 1, 0);
+    fetch_half(kt_first, 1);
+    stash_half(kt_first & 1, 1);
   }
   __syncthreads();
 
-  for (int kt = 0; kt < n_kt; ++kt) {
+  for (int kt = kt_first; kt < n_kt; ++kt) {
     const int stage = kt & 1;
     const bool more = kt + 1 < n_kt;
     const bool staged = more && window_ok(kt + 1);  // next tile fetched in halves during this one
@@ -712,6 +749,19 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
     const int row = row0_wg + wave * kRowsPerWave + cb * 16 + er;
     if (row >= nrows) continue;
     const int t = row / G;
+    if constexpr (kSplit) {
+      const int64_t pr = (int64_t)(q0 + t) * p.num_qo_heads + h * G + row % G;
+      if (q0 + t >= p.total_q) continue;  // past the partials: not a row of this call
+      if (kt_first == 0 && gq == 0) p.part_count[pr] = parts;
+      if (parts > 1) {
+        const int64_t slot = (int64_t)(run - h * p.splits) * p.total_q * p.num_qo_heads + pr;
+        if (gq == 0) p.part_ml[slot] = float2{m_run[cb], l_tot};
+        float* po = p.part_o + slot * D + 4 * gq;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(po + 16 * n) = o[cb][n];
+        continue;
+      }
+    }
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     const int64_t orr = grid_row(p, q0 + t);
     if (orr < 0) continue;
@@ -730,6 +780,60 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
 // Rows of every sequence with no key to attend (n_new > 0 but L = 0 cannot occur
 // with a consistent plan; sequences with n_new = 0 have no rows) need no pass.
 
+// Log-sum-exp merge of a split call's runs: D / 4 lanes per (token, query head) row, one
+// float4 each. Rows of one run are already in `out`.
+template <typename T, int D>
+__global__ void __launch_bounds__(256) prefill_merge_kernel(PrefillParams p) {
+  constexpr int kLanes = D / 4;
+  const int64_t rows = p.total_q * p.num_qo_heads;
+  const int64_t pr = (int64_t)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
+  if (pr >= rows) return;
+  const int t = (int)(pr / p.num_qo_heads);
+  if (t >= p.qo_indptr[p.batch]) return;  // a row of no sequence: nothing was left for it
+  // Every lane of a 16-lane group loads two runs' (max, sum) together with the count, so
+  // the row takes two rounds of loads whatever its runs (run by run, 17 runs took 20 us).
+  const int s_lane = threadIdx.x & 15;
+  float2 ml[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) ml[i] = p.part_ml[min(s_lane + 16 * i, p.splits - 1) * rows + pr];
+  const int parts = min(p.part_count[pr], p.splits);
+  if (parts <= 1) return;
+  const int64_t orr = grid_row(p, t);
+  if (orr < 0) return;
+  const int c = 4 * (threadIdx.x % kLanes);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (s_lane + 16 * i >= parts) ml[i] = float2{-INFINITY, 0.f};
+  float m_all = fmaxf(ml[0].x, ml[1].x);
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) m_all = fmaxf(m_all, __shfl_xor(m_all, off, 16));
+  float f[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) f[i] = ml[i].y == 0.f ? 0.f : fast_exp2(ml[i].x - m_all);  // 0: no key of the run seen
+  float l = fmaf(f[0], ml[0].y, f[1] * ml[1].y);
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) l += __shfl_xor(l, off, 16);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < parts; s0 += 8) {
+    f32x4 o[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      o[i] = *reinterpret_cast<const f32x4*>(p.part_o + (min(s0 + i, parts - 1) * rows + pr) * D + c);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (s0 + i >= parts) break;
+      const float fs = __shfl(s0 + i < 16 ? f[0] : f[1], (s0 + i) & 15, 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(fs, o[i][e], acc[e]);
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  u16x4 w;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = T::from_f32(acc[i] * inv);
+  *reinterpret_cast<u16x4*>(p.out + orr * p.out_stride + (pr - (int64_t)t * p.num_qo_heads) * D + c) = w;
+}
+
 inline int64_t grid_tiles(int64_t total_q, int32_t batch, int group, int rows_wg) {
   return (total_q * group + rows_wg - 1) / rows_wg + batch;
 }
@@ -738,8 +842,37 @@ template <typename T, int D>
 int launch_prefill(const PrefillParams& p, hipStream_t s) {
   // D = 64, 128: two column blocks (32 rows) per wave, 8 waves: measured faster than
   // four per wave at one wave per SIMD (chunk 3584..4095 of 8 x 4096: 276 vs 338 us)
-  paged_prefill_kernel<T, D><<<dim3((unsigned)(8 * p.per_xcd)), 64 * PrefillTile<D>::kWaves, 0, s>>>(p);
-  return check_launch("paged_prefill");
+  const dim3 grid((unsigned)(8 * p.per_xcd));
+  constexpr int kThreads = 64 * PrefillTile<D>::kWaves;
+  if (p.splits == 1) {
+    paged_prefill_kernel<T, D, false><<<grid, kThreads, 0, s>>>(p);
+    return check_launch("paged_prefill");
+  }
+  paged_prefill_kernel<T, D, true><<<grid, kThreads, 0, s>>>(p);
+  const int rc = check_launch("paged_prefill");
+  if (rc) return rc;
+  const int64_t rows = p.total_q * p.num_qo_heads;
+  prefill_merge_kernel<T, D><<<dim3((unsigned)((rows * (D / 4) + 255) / 256)), 256, 0, s>>>(p);
+  return check_launch("paged_prefill merge");
+}
+
+// Runs of keys per row tile. A workgroup takes a CU (its LDS), so a call of fewer than
+// half kCUs workgroups leaves CUs idle for as long as one workgroup walks its keys: its
+// tiles' keys are cut so that the workgroups fill the CUs once.
+int prefill_splits(int64_t total_q, int32_t batch, int32_t max_q, int group, int32_t num_kv_heads, int rows_wg) {
+  int64_t tiles = (total_q * group + rows_wg - 1) / rows_wg;  // at least this many
+  if (max_q > 0 && (int64_t)max_q * batch == total_q)         // a uniform batch: exactly
+    tiles = batch * (((int64_t)max_q * group + rows_wg - 1) / rows_wg);
+  const int64_t wgs = tiles * num_kv_heads;
+  const int64_t s = kCUs / (wgs < 1 ? 1 : wgs);
+  return (int)(s < 1 ? 1 : (s > kMaxSplits ? kMaxSplits : s));
+}
+
+// Partials of `splits` runs of total_q x Hq rows: part_count, part_ml, part_o.
+size_t split_bytes(int64_t rows, int splits, int head_dim) {
+  const size_t count = ((size_t)rows * 4 + 255) / 256 * 256;
+  const size_t ml = ((size_t)rows * splits * 8 + 255) / 256 * 256;
+  return 256 + count + ml + (size_t)rows * splits * head_dim * 4;
 }
 
 }  // namespace
@@ -750,12 +883,14 @@ using namespace nslg;
 extern "C" size_t nslg_paged_prefill_workspace_size(int32_t batch, int32_t num_qo_heads,
                                                     int32_t head_dim, int64_t total_q,
                                                     int32_t max_q) {
-  (void)batch;
-  (void)num_qo_heads;
-  (void)head_dim;
-  (void)total_q;
   (void)max_q;
-  return 256;  // the prefill kernel keeps all state on chip
+  if (batch <= 0 || num_qo_heads <= 0 || head_dim <= 0 || total_q <= 0) return 256;
+  // an upper bound of the runs of keys a call of this shape takes (whatever its KV heads)
+  const int64_t rows = total_q * num_qo_heads;
+  const int rows_wg = rows_per_wg(head_dim);
+  const int64_t s = kCUs / ((rows + rows_wg - 1) / rows_wg);
+  if (s < 2) return 256;  // one run: all state is kept on chip
+  return split_bytes(rows, (int)(s > kMaxSplits ? kMaxSplits : s), head_dim);
 }
 
 namespace {
@@ -765,8 +900,8 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
                  int64_t num_pages, int32_t page_size, const int32_t* kv_indptr, const int32_t* kv_indices,
                  const int32_t* kv_last_page_len, int32_t batch, int32_t num_qo_heads, int32_t num_kv_heads,
                  int32_t head_dim, float sm_scale, int32_t dtype, void* out, int64_t out_stride,
-                 nslg_stream_t stream, const void* k_new = nullptr, int64_t k_new_stride = 0,
-                 const void* v_new = nullptr, int64_t v_new_stride = 0) {
+                 void* workspace, size_t workspace_bytes, nslg_stream_t stream, const void* k_new = nullptr,
+                 int64_t k_new_stride = 0, const void* v_new = nullptr, int64_t v_new_stride = 0) {
   if (batch < 0 || num_qo_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || page_size <= 0 ||
       num_pages <= 0 || total_q < 0)
     return fail(NSLG_EINVAL, "paged_prefill: bad sizes");
@@ -876,7 +1011,26 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
   const int64_t slots = by_round && round_slots > tiles ? round_slots : tiles;
   if (slots * num_kv_heads > 0x7fffffff) return fail(NSLG_EUNSUPPORTED, "paged_prefill: too many rows");
   p.row_tiles = (int32_t)slots;
-  p.num_work = (int32_t)(slots * num_kv_heads);
+  p.total_q = total_q;
+  p.splits = 1;
+  p.part_o = nullptr;
+  p.part_ml = nullptr;
+  p.part_count = nullptr;
+  if (workspace && total_q > 0) {
+    int s = prefill_splits(total_q, batch, max_q, group, num_kv_heads, rows_wg);
+    const int64_t rows = total_q * num_qo_heads;
+    while (s > 1 && split_bytes(rows, s, head_dim) > workspace_bytes) --s;
+    if (s > 1) {
+      char* ws = (char*)(((uintptr_t)workspace + 255) / 256 * 256);  // (split_bytes has room for this)
+      p.splits = s;
+      p.part_count = (int32_t*)ws;
+      ws += ((size_t)rows * 4 + 255) / 256 * 256;
+      p.part_ml = (float2*)ws;
+      ws += ((size_t)rows * s * 8 + 255) / 256 * 256;
+      p.part_o = (float*)ws;
+    }
+  }
+  p.num_work = (int32_t)(slots * num_kv_heads * p.splits);
   p.q_rows = q_rows;
   p.grid_width = grid_width;
   p.pad_work = q_rows ? batch : 0;
@@ -917,11 +1071,9 @@ extern "C" int nslg_paged_prefill(const void* q, int64_t q_stride, const int32_t
                                   int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
                                   float sm_scale, int32_t dtype, void* out, int64_t out_stride,
                                   void* workspace, size_t workspace_bytes, nslg_stream_t stream) {
-  (void)workspace;
-  (void)workspace_bytes;
   return prefill_impl(q, q_stride, qo_indptr, nullptr, 0, total_q, max_q, k_pool, v_pool, num_pages, page_size,
                       kv_indptr, kv_indices, kv_last_page_len, batch, num_qo_heads, num_kv_heads, head_dim, sm_scale,
-                      dtype, out, out_stride, stream);
+                      dtype, out, out_stride, workspace, workspace_bytes, stream);
 }
 
 extern "C" int nslg_paged_prefill_grid(const void* q, int64_t q_stride, const int32_t* qo_indptr,
@@ -933,12 +1085,10 @@ extern "C" int nslg_paged_prefill_grid(const void* q, int64_t q_stride, const in
                                        int32_t head_dim, float sm_scale, int32_t dtype, void* out,
                                        int64_t out_stride, void* workspace, size_t workspace_bytes,
                                        nslg_stream_t stream) {
-  (void)workspace;
-  (void)workspace_bytes;
   if (batch > 0 && !q_rows) return fail(NSLG_EINVAL, "paged_prefill_grid: null q_rows");
   return prefill_impl(q, q_stride, qo_indptr, q_rows, grid_width, total_q, max_q, k_pool, v_pool, num_pages,
                       page_size, kv_indptr, kv_indices, kv_last_page_len, batch, num_qo_heads, num_kv_heads,
-                      head_dim, sm_scale, dtype, out, out_stride, stream);
+                      head_dim, sm_scale, dtype, out, out_stride, workspace, workspace_bytes, stream);
 }
 
 extern "C" int nslg_paged_prefill_append(const void* q, int64_t q_stride, const int32_t* qo_indptr,
@@ -951,10 +1101,9 @@ extern "C" int nslg_paged_prefill_append(const void* q, int64_t q_stride, const 
                                          int32_t head_dim, float sm_scale, int32_t dtype, void* out,
                                          int64_t out_stride, void* workspace, size_t workspace_bytes,
                                          nslg_stream_t stream) {
-  (void)workspace;
-  (void)workspace_bytes;
   if (batch > 0 && total_q > 0 && (!k_new || !v_new)) return fail(NSLG_EINVAL, "paged_prefill_append: null k_new/v_new");
   return prefill_impl(q, q_stride, qo_indptr, q_rows, grid_width, total_q, max_q, k_pool, v_pool, num_pages,
                       page_size, kv_indptr, kv_indices, kv_last_page_len, batch, num_qo_heads, num_kv_heads,
-                      head_dim, sm_scale, dtype, out, out_stride, stream, k_new, k_new_stride, v_new, v_new_stride);
+                      head_dim, sm_scale, dtype, out, out_stride, workspace, workspace_bytes, stream, k_new, k_new_stride, v_new,
+                      v_new_stride);
 }

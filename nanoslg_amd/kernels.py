@@ -890,14 +890,43 @@ class DecodeLaunch:
 _PREFILL_WS: Dict[Tuple[int, int, int, int, int], int] = {}  # nslg_paged_prefill_workspace_size by call shape
 
 
+# Keys of the longest sequence from which a prefill call gets a workspace, so that the
+# library may cut its row tiles' keys into runs. Measured at 32/8 heads x 128, one
+# sequence: 512 new tokens from zero 25.7 us either way (bf16 31.1 -> 27.5), 256 from
+# zero 17.7 us in one run and 20.4 in runs, 16 over 512 18.8 and 14.4.
+PREFILL_SPLIT_KEYS = 512
+
+
+def _prefill_workspace(q, B, Hq, D, total_q, max_q, max_kv):
+    """(owner, address, bytes) of the partials of a prefill call whose longest sequence has
+    max_kv keys; (None, None, 0) where the call takes its keys in one run. From the caching
+    allocator on the current stream, and not the cache's workspace: one cache's prefills
+    may run on another stream than its decodes."""
+    if max_kv < PREFILL_SPLIT_KEYS:
+        return None, None, 0
+    key = (B, Hq, D, total_q, max_q)
+    need = _PREFILL_WS.get(key)
+    if need is None:  # a pure function of the call shape: asked once per shape
+        need = int(_lib.load().nslg_paged_prefill_workspace_size(*key))
+        if len(_PREFILL_WS) > 4096:
+            _PREFILL_WS.clear()
+        _PREFILL_WS[key] = need
+    if need <= 256:
+        return None, None, 0
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+    return ws, ws.data_ptr(), need
+
+
 def _paged_prefill_layer(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int, max_q: int,
                          k_layer: torch.Tensor, v_layer: torch.Tensor, kv_indptr: torch.Tensor,
                          kv_indices: torch.Tensor, kv_last_page_len: torch.Tensor, workspace: Workspace,
-                         q_rows: Optional[torch.Tensor] = None, grid_width: int = 0) -> torch.Tensor:
-    """paged_prefill for the cache manager: its pool layer, plan (int32 arrays on the
-    pool's device, qo_indptr and kv_indptr of B + 1 entries) and workspace are taken
-    as they are; the caller's q gets paged_prefill's checks (a q that fails one goes
-    through paged_prefill, which raises its error). Default scale 1/sqrt(D)."""
+                         q_rows: Optional[torch.Tensor] = None, grid_width: int = 0,
+                         max_kv: int = 0) -> torch.Tensor:
+    """paged_prefill for the cache manager: its pool layer and plan (int32 arrays on the
+    pool's device, qo_indptr and kv_indptr of B + 1 entries) are taken as they are; the
+    caller's q gets paged_prefill's checks (a q that fails one goes through paged_prefill,
+    which raises its error). Default scale 1/sqrt(D). max_kv: the longest sequence's keys,
+    new ones included (0: its keys are taken in one run)."""
     dev, dt = k_layer.get_device(), k_layer.dtype
     P, ps, Hkv, D = k_layer.shape
     B = kv_indptr.numel() - 1
@@ -909,13 +938,7 @@ def _paged_prefill_layer(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int,
     T, Hq = q.shape[0], q.shape[1]
     out = torch.empty((T, Hq, D), dtype=dt, device=q.device)
     fast = _lib.fast()
-    key = (B, Hq, D, int(total_q), int(max_q))
-    need = _PREFILL_WS.get(key)
-    if need is None:  # a pure function of the call shape: asked once per shape
-        need = _PREFILL_WS[key] = int(_lib.load().nslg_paged_prefill_workspace_size(*key))
-        if len(_PREFILL_WS) > 4096:
-            _PREFILL_WS.clear()
-    ws = workspace.get(need)
+    ws, ws_ptr, ws_bytes = _prefill_workspace(q, B, Hq, D, int(total_q), int(max_q), max_kv)
     stream = _stream(k_layer)
     scale = 1.0 / math.sqrt(D)
     if q_rows is not None:
@@ -923,13 +946,13 @@ def _paged_prefill_layer(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int,
                                      int(grid_width), int(total_q), int(max_q), k_layer.data_ptr(),
                                      v_layer.data_ptr(), P, ps, kv_indptr.data_ptr(), kv_indices.data_ptr(),
                                      kv_last_page_len.data_ptr(), B, Hq, Hkv, D, scale, _DTYPE_CODE[dt],
-                                     out.data_ptr(), Hq * D, ws.data_ptr(), ws.numel(), stream)
+                                     out.data_ptr(), Hq * D, ws_ptr, ws_bytes, stream)
         _lib.check(rc, "nslg_paged_prefill_grid")
         return out
     rc = fast.paged_prefill(q.data_ptr(), q.stride(0), qo_indptr.data_ptr(), int(total_q), int(max_q),
                             k_layer.data_ptr(), v_layer.data_ptr(), P, ps, kv_indptr.data_ptr(),
                             kv_indices.data_ptr(), kv_last_page_len.data_ptr(), B, Hq, Hkv, D, scale, _DTYPE_CODE[dt],
-                            out.data_ptr(), Hq * D, ws.data_ptr(), ws.numel(), stream)
+                            out.data_ptr(), Hq * D, ws_ptr, ws_bytes, stream)
     _lib.check(rc, "nslg_paged_prefill")
     return out
 
@@ -938,11 +961,11 @@ def _paged_prefill_append_layer(q: torch.Tensor, qo_indptr: torch.Tensor, total_
                                 k_new: torch.Tensor, v_new: torch.Tensor, k_layer: torch.Tensor,
                                 v_layer: torch.Tensor, kv_indptr: torch.Tensor, kv_indices: torch.Tensor,
                                 kv_last_page_len: torch.Tensor, workspace: Workspace,
-                                q_rows: Optional[torch.Tensor] = None, grid_width: int = 0
-                                ) -> Optional[torch.Tensor]:
-    """nslg_paged_prefill_append for the cache manager (its pool layer, plan and
-    workspace taken as they are): the forward's K/V rows written and its queries
-    attended in one launch. None, with nothing launched, where the one launch does not
+                                q_rows: Optional[torch.Tensor] = None, grid_width: int = 0,
+                                max_kv: int = 0) -> Optional[torch.Tensor]:
+    """nslg_paged_prefill_append for the cache manager (its pool layer and plan taken as
+    they are, max_kv as in _paged_prefill_layer): the forward's K/V rows written and its
+    queries attended in one launch. None, with nothing launched, where the one launch does not
     apply (fp32 pools, q / k_new / v_new not rows of a 16-bit forward at one 16-byte
     stride each): the caller then appends and runs _paged_prefill_layer, whose checks
     raise any error."""
@@ -972,19 +995,13 @@ def _paged_prefill_append_layer(q: torch.Tensor, qo_indptr: torch.Tensor, total_
         return None
     Hq = q.shape[1]
     out = torch.empty((n, Hq, D), dtype=dt, device=q.device)
-    key = (B, Hq, D, int(total_q), int(max_q))
-    need = _PREFILL_WS.get(key)
-    if need is None:
-        need = _PREFILL_WS[key] = int(_lib.load().nslg_paged_prefill_workspace_size(*key))
-        if len(_PREFILL_WS) > 4096:
-            _PREFILL_WS.clear()
-    ws = workspace.get(need)
+    ws, ws_ptr, ws_bytes = _prefill_workspace(q, B, Hq, D, int(total_q), int(max_q), max_kv)
     rc = _lib.fast().paged_prefill_append(
         q.data_ptr(), q.stride(0), qo_indptr.data_ptr(), None if q_rows is None else q_rows.data_ptr(),
         int(grid_width), int(total_q), int(max_q), k_new.data_ptr(), strides[0], v_new.data_ptr(), strides[1],
         k_layer.data_ptr(), v_layer.data_ptr(), P, ps, kv_indptr.data_ptr(), kv_indices.data_ptr(),
         kv_last_page_len.data_ptr(), B, Hq, Hkv, D, 1.0 / math.sqrt(D), _DTYPE_CODE[dt], out.data_ptr(), Hq * D,
-        ws.data_ptr(), ws.numel(), _stream(k_layer))
+        ws_ptr, ws_bytes, _stream(k_layer))
     _lib.check(rc, "nslg_paged_prefill_append")
     return out
 
@@ -1025,16 +1042,17 @@ def paged_prefill_append(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int,
         raise ValueError("paged_prefill_append: qo_indptr must have B+1 entries and q at least total_q rows")
     out = torch.empty((T, Hq, D), dtype=q.dtype, device=q.device)
     lib = _lib.load()
-    need = int(lib.nslg_paged_prefill_workspace_size(B, Hq, D, int(total_q), int(max_q)))
-    ws = (workspace or Workspace(q.device)).get(need)
+    # the average sequence's table stands for the longest one (its length is on the device)
+    max_kv = kv_indices.numel() * ps // max(B, 1)
+    ws, ws_ptr, ws_bytes = _prefill_workspace(q, B, Hq, D, int(total_q), int(max_q), max_kv)
     scale = (1.0 / math.sqrt(D)) if sm_scale is None else float(sm_scale)
     rc = lib.nslg_paged_prefill_append(q.data_ptr(), q.stride(0), qo_indptr.data_ptr(),
                                        None if q_rows is None else q_rows.data_ptr(), int(grid_width),
                                        int(total_q), int(max_q), k_new.data_ptr(), ks, v_new.data_ptr(), vs,
                                        k_layer.data_ptr(), v_layer.data_ptr(), P, ps, kv_indptr.data_ptr(),
                                        kv_indices.data_ptr(), kv_last_page_len.data_ptr(), B, Hq, Hkv, D, scale,
-                                       dtype_code(q.dtype), out.data_ptr(), out.stride(0), ws.data_ptr(),
-                                       ws.numel(), _stream(q))
+                                       dtype_code(q.dtype), out.data_ptr(), out.stride(0), ws_ptr, ws_bytes,
+                                       _stream(q))
     _lib.check(rc, "nslg_paged_prefill_append")
     return out
 
@@ -1074,21 +1092,21 @@ def paged_prefill(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int, max_q:
                                  or out.stride(2) != 1 or out.stride(1) != D or out.dtype != q.dtype):
         raise ValueError("paged_prefill: out must be the grid's [B * grid_width, Hq, D] rows")
     lib = _lib.load()
-    need = int(lib.nslg_paged_prefill_workspace_size(B, Hq, D, int(total_q), int(max_q)))
-    ws = (workspace or Workspace(q.device)).get(need)
+    # the average sequence's table stands for the longest one (its length is on the device)
+    max_kv = kv_indices.numel() * ps // max(B, 1)
+    ws, ws_ptr, ws_bytes = _prefill_workspace(q, B, Hq, D, int(total_q), int(max_q), max_kv)
     scale = (1.0 / math.sqrt(D)) if sm_scale is None else float(sm_scale)
     if q_rows is not None:
         rc = lib.nslg_paged_prefill_grid(q.data_ptr(), q.stride(0), qo_indptr.data_ptr(), q_rows.data_ptr(),
                                          int(grid_width), int(total_q), int(max_q), k_layer.data_ptr(),
                                          v_layer.data_ptr(), P, ps, kv_indptr.data_ptr(), kv_indices.data_ptr(),
                                          kv_last_page_len.data_ptr(), B, Hq, Hkv, D, scale, dtype_code(q.dtype),
-                                         out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(), _stream(q))
+                                         out.data_ptr(), out.stride(0), ws_ptr, ws_bytes, _stream(q))
         _lib.check(rc, "nslg_paged_prefill_grid")
         return out
     rc = lib.nslg_paged_prefill(q.data_ptr(), q.stride(0), qo_indptr.data_ptr(), int(total_q), int(max_q),
                                 k_layer.data_ptr(), v_layer.data_ptr(), P, ps, kv_indptr.data_ptr(),
                                 kv_indices.data_ptr(), kv_last_page_len.data_ptr(), B, Hq, Hkv, D, scale,
-                                dtype_code(q.dtype), out.data_ptr(), out.stride(0), ws.data_ptr(),
-                                ws.numel(), _stream(q))
+                                dtype_code(q.dtype), out.data_ptr(), out.stride(0), ws_ptr, ws_bytes, _stream(q))
     _lib.check(rc, "nslg_paged_prefill")
     return out

@@ -53,6 +53,11 @@ def _default_kernels():
     return kernels
 
 
+def _key_bound(kernels, max_kv: int) -> Dict[str, int]:
+    """The longest sequence's keys, for prefill calls that can cut them into runs."""
+    return {"max_kv": max_kv} if hasattr(kernels, "PREFILL_SPLIT_KEYS") else {}
+
+
 def _host_planner():
     from . import _lib
     return _lib.host().plan_forward
@@ -1229,20 +1234,21 @@ class PagedCacheContext(CacheContext):
         B, S = q.shape[0], q.shape[1]
         Hq, D = q.shape[2], q.shape[3]
         q_grid = q.reshape(B * S, Hq, D)
+        bound = _key_bound(kern, self.max_kv_len)
         if k_new is not None:
             uniform = self._uniform_rows and S == self._iw
             o = kern._paged_prefill_append_layer(
                 q_grid, plan.qo_indptr, plan.total_q, self._max_q, k_new, v_new, k_layer, v_layer, plan.indptr,
                 plan.indices, plan.lpl, cache.workspace, q_rows=None if uniform else plan.rows_for(S),
-                grid_width=0 if uniform else S)
+                grid_width=0 if uniform else S, **bound)
             return None if o is None else o.view(B, S, Hq * D)
         if self._uniform_rows and S == self._iw:  # every grid row is a token: the ragged rows themselves
             o = kern._paged_prefill_layer(q_grid, plan.qo_indptr, plan.total_q, self._max_q, k_layer, v_layer,
-                                          plan.indptr, plan.indices, plan.lpl, cache.workspace)
+                                          plan.indptr, plan.indices, plan.lpl, cache.workspace, **bound)
         else:  # padded or ragged: the kernel reads and writes the grid rows (pad rows zero)
             o = kern._paged_prefill_layer(q_grid, plan.qo_indptr, plan.total_q, self._max_q, k_layer, v_layer,
                                           plan.indptr, plan.indices, plan.lpl, cache.workspace,
-                                          q_rows=plan.rows_for(S), grid_width=S)
+                                          q_rows=plan.rows_for(S), grid_width=S, **bound)
         return o.view(B, S, Hq * D)
 
     # ---- introspection used by tests and the bench -------------------------------------
@@ -1836,7 +1842,8 @@ class ContiguousCacheContext(CacheContext):
             o = cache.kernels._paged_prefill_append_layer(
                 q.reshape(B * S, q.shape[2], q.shape[3]), plan.qo_indptr, plan.total_q, self._max_q, k_new, v_new,
                 k_layer, v_layer, plan.indptr, plan.indices, plan.lpl, cache.workspace,
-                q_rows=None if uniform else plan.rows_for(S), grid_width=0 if uniform else S)
+                q_rows=None if uniform else plan.rows_for(S), grid_width=0 if uniform else S,
+                **_key_bound(cache.kernels, self.max_kv_len))
             if o is not None:
                 return o.view(B, S, -1)
         cache.kernels.append_kv(k_new, v_new, plan.slots_for(S), k_layer, v_layer)
@@ -1868,13 +1875,11 @@ class ContiguousCacheContext(CacheContext):
             return out.reshape(B, 1, -1)
         Hq, D = q.shape[2], q.shape[3]
         q_grid = q.reshape(B * S, Hq, D)
-        if self._uniform_rows and S == self._iw:  # every grid row is a token: the ragged rows themselves
-            o = kern.paged_prefill(q_grid, plan.qo_indptr, plan.total_q, self._max_q, k_layer, v_layer,
-                                   plan.indptr, plan.indices, plan.lpl, workspace=cache.workspace)
-        else:  # padded or ragged: the kernel reads and writes the grid rows (pad rows zero)
-            o = kern.paged_prefill(q_grid, plan.qo_indptr, plan.total_q, self._max_q, k_layer, v_layer,
-                                   plan.indptr, plan.indices, plan.lpl, workspace=cache.workspace,
-                                   q_rows=plan.rows_for(S), grid_width=S)
+        grid = {} if self._uniform_rows and S == self._iw else {"q_rows": plan.rows_for(S), "grid_width": S}
+        # (padded or ragged: the kernel reads and writes the grid rows, pad rows zero)
+        o = kern._paged_prefill_layer(q_grid, plan.qo_indptr, plan.total_q, self._max_q, k_layer, v_layer, plan.indptr,
+                                      plan.indices, plan.lpl, cache.workspace, **grid,
+                                      **_key_bound(kern, self.max_kv_len))
         return o.view(B, S, Hq * D)
 
 

@@ -1,0 +1,72 @@
+"""Prefill calls of few row tiles, whose keys are cut into runs and merged: against the
+oracle's fp32 attention within the attention tolerance, and the forward's K/V write of a
+cut call bit-identical to nslg_append_kv. Keys at the edges of key tiles, runs and page-id
+windows; sequences shorter than a run, without new tokens, and of one new token; padded
+grids; every head dim, GQA group 1, 4 and 16."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_kernels import ATOL, RTOL, _prefill_case
+
+DEV = "cuda:0"
+
+CASES = [  # lens, new tokens, Hq, Hkv, D, page size
+    ([512], [1], 32, 8, 128, 16),               # the shortest sequence that is cut
+    ([513], [17], 32, 8, 128, 16),              # a last run of one key
+    ([4096 + 31], [31], 8, 8, 128, 1),          # G = 1, 32 runs across two page-id windows
+    ([6000, 300, 900], [33, 0, 5], 32, 8, 128, 16),
+    ([1600, 1500], [150, 70], 16, 1, 128, 48),  # G = 16
+    ([2100], [300], 32, 8, 64, 16),
+    ([700, 3000], [1, 129], 16, 4, 256, 16),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_prefill_in_runs_matches_oracle(case, dtype, monkeypatch):
+    from nanoslg_amd import kernels as K
+    lens, news, Hq, Hkv, D, ps = CASES[case]
+    got = []
+    orig = K._prefill_workspace
+    monkeypatch.setattr(K, "_prefill_workspace", lambda *a: got.append(orig(*a)) or got[-1])
+    out, ref = _prefill_case(lens, news, Hq, Hkv, D, ps, dtype, seed=700 + case)
+    assert got and got[0][2] > 256  # the call had room for runs
+    torch.testing.assert_close(out, ref, atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grid", [False, True])
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 128), (torch.bfloat16, 64), (torch.float16, 256)])
+def test_prefill_in_runs_writes_the_new_rows(dtype, D, grid):
+    """The fused write of a call cut into runs: pool bytes as append_kv leaves them, the
+    result that of append_kv then prefill; tokens across a run's end and a page's."""
+    from nanoslg_amd import kernels as K
+    Hq, Hkv, ps, start, news = 16, 4, 16, [1000, 1270], [90, 25]
+    g = torch.Generator().manual_seed(90 + D)
+    npg = [-(-(s + n) // ps) for s, n in zip(start, news)]
+    P, W = sum(npg) + 2, max(news) + 3
+    ids = np.random.default_rng(9).permutation(np.arange(1, P))[:sum(npg)].astype(np.int32)
+    indptr = np.array([0, npg[0], sum(npg)], np.int32)
+    lpl = np.array([(s + n - 1) % ps + 1 for s, n in zip(start, news)], np.int32)
+    qo = np.array([0, news[0], sum(news)], np.int32)
+    rows = np.concatenate([b * W + 3 + np.arange(n) for b, n in enumerate(news)]).astype(np.int32)
+    slots = np.full(2 * W, -1, np.int32)
+    for b in range(2):
+        pos = start[b] + np.arange(news[b])
+        slots[b * W + 3 + np.arange(news[b])] = ids[indptr[b] + pos // ps] * ps + pos % ps
+    n = 2 * W if grid else sum(news)
+    if not grid:
+        slots = slots[rows]
+    q, k, v = (torch.randn(n, h, D, generator=g).to(dtype).to(DEV) for h in (Hq, Hkv, Hkv))
+    k1, v1 = (torch.randn(P, ps, Hkv, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+    k2, v2 = k1.clone(), v1.clone()
+    d = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    plan = (d(indptr), d(ids), d(lpl))
+    kw = dict(q_rows=d(rows), grid_width=W) if grid else {}
+    o1 = K.paged_prefill_append(q, d(qo), sum(news), max(news), k, v, k1, v1, *plan, **kw)
+    K.append_kv(k, v, d(slots), k2, v2)
+    o2 = K.paged_prefill(q, d(qo), sum(news), max(news), k2, v2, *plan, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(o1, o2)
