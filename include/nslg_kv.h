@@ -143,9 +143,9 @@ int nslg_gather_kv(const void* k_pool, const void* v_pool, int64_t num_pages,
  *                     another forward (a wrong record gives wrong results, though
  *                     every access stays inside the block table and the pool).
  * Query head h reads KV head h / (Hq/Hkv). Supported: f16, bf16 (MFMA, split-K as
- * above) and f32 (a VALU kernel, one workgroup per 16 query rows of a sequence and
- * KV head and key split, then an fp32 merge, for caches kept in fp32 such as the
- * contiguous backend of an fp32 model, kv_cache.py:227-322); D in {64, 128, 256};
+ * above) and f32 (fp32 MFMA, one workgroup per sequence, KV head and run of keys,
+ * then an fp32 merge, for caches kept in fp32 such as the contiguous backend of an
+ * fp32 model, kv_cache.py:227-322); D in {64, 128, 256};
  * 1 <= Hq/Hkv <= 16. A sequence with no tokens gets zeros.
  * The first f16/bf16 call of a (dtype, head_dim, page_size) variant on a device
  * (or the first workspace-size query for it) queries the device's occupancy
@@ -353,7 +353,7 @@ int nslg_paged_decode_grouped_rope_append(
  *               keys into runs and merges them (a second launch). Null or smaller:
  *               fewer runs, or one and no use of the workspace
  * Supported: f16, bf16 with D in {64, 128, 256} (MFMA); f32 with D in {64, 128,
- * 256} (the VALU kernel of nslg_paged_decode's f32 path); 1 <= Hq/Hkv <= 16.
+ * 256} (fp32 MFMA, attn_f32.hip); 1 <= Hq/Hkv <= 16.
  */
 size_t nslg_paged_prefill_workspace_size(int32_t batch, int32_t num_qo_heads,
                                          int32_t head_dim, int64_t total_q,

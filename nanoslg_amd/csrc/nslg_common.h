@@ -211,15 +211,25 @@ struct AttnF32Args {
   float scale;                 // softmax scale, natural-exponent units
   float* out;
   int64_t out_stride;
-  int32_t row_tiles;           // set by attention_f32
-  int32_t splits;              // key ranges per row tile (1: no partials)
-  float* part_o;               // splits > 1: [total_q, Hq, splits, D] partial outputs
-  float* part_ml;              // splits > 1: [total_q, Hq, splits, 2] running max and sum
+  int64_t total_q;             // query tokens (batch for decode)
+  // decode: the step's new rows (null: none), sequence b's token L_b - 1, written into
+  // the pool by the call; strides in elements between batch rows
+  const float* k_new = nullptr;
+  const float* v_new = nullptr;
+  int64_t k_new_stride = 0;
+  int64_t v_new_stride = 0;
+  int32_t splits;              // runs of keys per row tile (1: no partials)
+  void* workspace = nullptr;   // splits > 1: attention_f32_workspace bytes
+  int32_t row_tiles = 0;       // these are set by attention_f32
+  float* part_o = nullptr;     // [splits, total_q, Hq, D] partial outputs
+  float* part_ml = nullptr;    // [splits, total_q, Hq, 2] running max and sum
 };
-// Launch on stream s; total_q = number of query tokens (B for decode).
-int attention_f32(const AttnF32Args& a, int64_t total_q, int32_t head_dim, hipStream_t s);
-// Key splits for a decode batch, and the workspace they need.
-int attention_f32_splits(int64_t batch, int64_t total_tokens);
+// Launch on stream s (decode if qo_indptr is null, else prefill).
+int attention_f32(const AttnF32Args& a, int32_t head_dim, hipStream_t s);
+// Runs of keys for a decode batch of at most total_tokens keys in all, for a prefill of
+// total_q rows with that workspace, and the workspace they need.
+int attention_f32_decode_splits(int64_t batch, int32_t num_kv_heads, int64_t total_tokens);
+int attention_f32_prefill_splits(int64_t total_q, int32_t num_qo_heads, size_t workspace_bytes, int32_t head_dim);
 size_t attention_f32_workspace(int64_t total_q, int32_t num_qo_heads, int32_t head_dim, int splits);
 
 }  // namespace nslg

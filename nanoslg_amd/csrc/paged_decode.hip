@@ -1110,27 +1110,6 @@ int launch_decode(const DecodeParams& p, const MergeParams& mp, const GroupArgs<
   return check_launch("paged_decode_merge");
 }
 
-// New rows of an fp32 decode call (whose attention kernel has no folded write):
-// grid (batch, 2), workgroup b writes sequence b's K (y = 0) or V (y = 1) row as
-// its token L_b - 1, the slot found through its block table. 4-byte words.
-__global__ void __launch_bounds__(256)
-write_last_rows_kernel(const uint32_t* __restrict__ k_new, const uint32_t* __restrict__ v_new,
-                       int64_t k_stride_words, int64_t v_stride_words, const int32_t* __restrict__ indptr,
-                       const int32_t* __restrict__ indices, const int32_t* __restrict__ last_len,
-                       int32_t page_size, int64_t num_pages, int32_t row_words, uint32_t* __restrict__ k_pool,
-                       uint32_t* __restrict__ v_pool) {
-  const int b = blockIdx.x;
-  const int len = seq_len_of(indptr, last_len, b, page_size);
-  if (len <= 0) return;
-  const int tok = len - 1;
-  const int pid = indices[indptr[b] + tok / page_size];
-  if (pid < 0 || (int64_t)pid >= num_pages) return;
-  const bool is_v = blockIdx.y != 0;
-  const uint32_t* src = is_v ? v_new + (int64_t)b * v_stride_words : k_new + (int64_t)b * k_stride_words;
-  uint32_t* dst = (is_v ? v_pool : k_pool) + ((int64_t)pid * page_size + tok % page_size) * row_words;
-  for (int i = threadIdx.x; i < row_words; i += blockDim.x) dst[i] = src[i];
-}
-
 inline size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Workspace: partials [max_chunks, slot_members, Hq, D] and [..., 2] fp32, then each
@@ -1232,28 +1211,21 @@ int decode_impl(const void* q, int64_t q_stride, const void* k_pool, const void*
       a.scale = sm_scale;
       a.out = (float*)out;
       a.out_stride = out_stride;
-      a.row_tiles = 0;
+      a.total_q = batch;
+      a.k_new = (const float*)nr.k;
+      a.v_new = (const float*)nr.v;
+      a.k_new_stride = nr.k_stride;
+      a.v_new_stride = nr.v_stride;
       // long sequences are split over keys; the partials go to the workspace
-      a.splits = attention_f32_splits(batch, total_pages * (int64_t)page_size);
-      a.part_o = nullptr;
-      a.part_ml = nullptr;
+      a.splits = attention_f32_decode_splits(batch, num_kv_heads, total_pages * (int64_t)page_size);
       if (a.splits > 1) {
         const size_t need = attention_f32_workspace(batch, num_qo_heads, head_dim, a.splits);
         if (!workspace || workspace_bytes < need)
           return fail(NSLG_EWORKSPACE, "paged_decode: workspace %zu < %zu bytes", workspace_bytes, need);
         if (((uintptr_t)workspace) & 255) return fail(NSLG_EINVAL, "paged_decode: workspace must be 256-byte aligned");
-        a.part_o = (float*)workspace;
-        a.part_ml = a.part_o + (int64_t)batch * num_qo_heads * a.splits * head_dim;
+        a.workspace = workspace;
       }
-      if (nr.k) {
-        const int row_words = num_kv_heads * head_dim;
-        write_last_rows_kernel<<<dim3(batch, 2), row_words < 256 ? 64 : 256, 0, as_stream(stream)>>>(
-            (const uint32_t*)nr.k, (const uint32_t*)nr.v, nr.k_stride, nr.v_stride, kv_indptr, kv_indices,
-            kv_last_page_len, page_size, num_pages, row_words, (uint32_t*)k_pool, (uint32_t*)v_pool);
-        const int rc = check_launch("paged_decode_append (rows)");
-        if (rc) return rc;
-      }
-      return attention_f32(a, batch, head_dim, as_stream(stream));
+      return attention_f32(a, head_dim, as_stream(stream));
     }
   }
   if (dtype != NSLG_F16 && dtype != NSLG_BF16)
@@ -1383,7 +1355,8 @@ extern "C" size_t nslg_paged_decode_workspace_size(int32_t batch, int32_t num_qo
   if (!shape_ok(batch, num_qo_heads, num_kv_heads, head_dim, total_pages, page_size)) return 0;
   if (dtype == NSLG_F32)  // partials of the key splits of the fp32 path
     return attention_f32_workspace(batch, num_qo_heads, head_dim,
-                                   attention_f32_splits(batch, total_pages * (int64_t)page_size));
+                                   attention_f32_decode_splits(batch, num_kv_heads,
+                                                               total_pages * (int64_t)page_size));
   const DecodeShape sh = shape_of<false>(dtype, head_dim, batch, num_kv_heads, total_pages * page_size, page_size);
   return workspace_bytes_for(sh, batch, num_qo_heads, head_dim, 1, 0);
 }

@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   }
   const int runs = p.num_kv_heads * p.splits;
   const int run = kSplit ? w % runs : w / p.row_tiles;  // (KV head, run of keys)
-  const int h = kSplit ? run / p.splits : run;
+  const int h = kSplit ? run % p.num_kv_heads : run;
   int b = 0, tile = 0;
   const int g = kSplit ? w / runs : w - run * p.row_tiles;
   // longest-first rounds when the host's round count covers every sequence (it came
@@ -280,7 +280,7 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   int parts = 1;
   if constexpr (kSplit) {
     // equal runs of key tiles, of at least kMinRun tiles each
-    const int split = run - h * p.splits;
+    const int split = run / p.num_kv_heads;  // (a head's runs, of unequal keys, on one XCD)
     const int per = max((n_kt + p.splits - 1) / p.splits, kMinRun);
     parts = max((n_kt + per - 1) / per, 1);
     if (split >= parts) return;
@@ -754,7 +754,7 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
       if (q0 + t >= p.total_q) continue;  // past the partials: not a row of this call
       if (kt_first == 0 && gq == 0) p.part_count[pr] = parts;
       if (parts > 1) {
-        const int64_t slot = (int64_t)(run - h * p.splits) * p.total_q * p.num_qo_heads + pr;
+        const int64_t slot = (int64_t)(run / p.num_kv_heads) * p.total_q * p.num_qo_heads + pr;
         if (gq == 0) p.part_ml[slot] = float2{m_run[cb], l_tot};
         float* po = p.part_o + slot * D + 4 * gq;
 #pragma unroll
@@ -943,13 +943,12 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
     a.scale = sm_scale;
     a.out = (float*)out;
     a.out_stride = out_stride;
-    a.row_tiles = 0;
+    a.total_q = total_q;
     a.q_rows = q_rows;
     a.grid_width = grid_width;
-    a.splits = 1;  // the query rows fill the GPU
-    a.part_o = nullptr;
-    a.part_ml = nullptr;
-    return attention_f32(a, total_q, head_dim, as_stream(stream));
+    a.workspace = workspace;
+    a.splits = workspace ? attention_f32_prefill_splits(total_q, num_qo_heads, workspace_bytes, head_dim) : 1;
+    return attention_f32(a, head_dim, as_stream(stream));
   }
   if (dtype != NSLG_F16 && dtype != NSLG_BF16)
     return fail(NSLG_EUNSUPPORTED, "paged_prefill: dtype %d", dtype);

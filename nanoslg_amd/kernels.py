@@ -20,8 +20,8 @@ _DTYPE_CODE = {torch.float16: _lib.NSLG_F16, torch.bfloat16: _lib.NSLG_BF16, tor
 # decode batches of other pools are decoded per sequence.
 GROUPED_DECODE_DTYPES = (torch.float16, torch.bfloat16)
 # head dims each pool dtype supports on every entry point a cache uses: decode, RoPE
-# append and prefill take 64, 128 and 256 (16-bit pools on the MFMA kernels, fp32
-# pools on the VALU attention kernel)
+# append and prefill take 64, 128 and 256 (16-bit pools on the 16-bit MFMA kernels, fp32
+# pools on the fp32 ones)
 HEAD_DIMS = {torch.float16: (64, 128, 256), torch.bfloat16: (64, 128, 256), torch.float32: (64, 128, 256)}
 
 

@@ -1,0 +1,62 @@
+"""The fp32 attention kernels at the edges of their tiles, waves, runs and pages, against
+the oracle's fp32 SDPA (within summation-order differences), and the decode's fused write
+of the new rows against append_kv."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_kernels import F32_TOL, _csr_random, _decode_case, _prefill_case
+
+DEV = "cuda:0"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,Hq,Hkv,D,ps", [
+    ([1, 15, 16, 17, 63, 64, 65, 0], 8, 2, 128, 16),   # one tile and its neighbours, one wave each and more
+    ([129, 4, 640, 1000], 16, 1, 128, 5),              # G = 16, tiles across pages
+    ([4500], 4, 4, 128, 1),                            # G = 1, 64 runs
+    ([70, 2000, 0, 33], 32, 8, 64, 48),
+    ([31, 900], 12, 2, 256, 16),
+    ([700] * 40, 8, 8, 128, 700),                      # whole slots, one run each
+])
+def test_f32_decode_edges(lens, Hq, Hkv, D, ps):
+    out, ref = _decode_case(lens, Hq, Hkv, D, ps, torch.float32, seed=800 + D + ps)
+    torch.testing.assert_close(out, ref, **F32_TOL)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,news,Hq,Hkv,D,ps", [
+    ([1, 16, 17, 33], [1, 16, 17, 2], 32, 8, 128, 16),     # row tiles of one token to one and a bit
+    ([100, 300, 64], [100, 0, 31], 12, 4, 128, 5),         # G = 3: tokens across waves; no new tokens
+    ([1200, 520], [40, 7], 8, 8, 128, 16),                 # runs of keys, merged
+    ([700], [300], 16, 1, 64, 1),                          # G = 16, one-token pages
+    ([90, 600], [90, 33], 16, 4, 256, 48),
+    ([530] * 24, [40] * 24, 32, 8, 128, 16),               # more workgroups than take two key groups
+])
+def test_f32_prefill_edges(lens, news, Hq, Hkv, D, ps):
+    out, ref = _prefill_case(lens, news, Hq, Hkv, D, ps, torch.float32, seed=820 + D + ps)
+    torch.testing.assert_close(out, ref, **F32_TOL)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_f32_decode_writes_the_new_rows(D):
+    """paged_decode_append on rows 4-byte aligned only: the pool as append_kv leaves it,
+    the result that of append_kv then paged_decode, bit for bit."""
+    from nanoslg_amd import kernels as K
+    Hq, Hkv, ps, lens = 8, 2, 16, [1, 16, 17, 64, 65, 900]
+    g = torch.Generator().manual_seed(D)
+    P = sum(-(-n // ps) for n in lens) + 2
+    _, (indptr, indices, lpl) = _csr_random(lens, ps, P, D)
+    slots = np.array([indices[indptr[b + 1] - 1] * ps + (n - 1) % ps for b, n in enumerate(lens)], np.int32)
+    rows = torch.randn(2, len(lens), Hkv * D + 1, generator=g).to(DEV)
+    k, v = (x[:, 1:].unflatten(1, (Hkv, D)) for x in rows)  # rows at an odd stride, off 16 bytes
+    q = torch.randn(len(lens), Hq, D, generator=g).to(DEV)
+    k1, v1 = (torch.randn(P, ps, Hkv, D, generator=g).to(DEV) for _ in range(2))
+    k2, v2 = k1.clone(), v1.clone()
+    plan = tuple(torch.from_numpy(a).to(DEV) for a in (indptr, indices, lpl)) + (int(indptr[-1]),)
+    o1 = K.paged_decode_append(q, k, v, k1, v1, *plan)
+    K.append_kv(k, v, torch.from_numpy(slots).to(DEV), k2, v2)
+    o2 = K.paged_decode(q, k2, v2, *plan)
+    torch.cuda.synchronize()
+    assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(o1, o2)
