@@ -43,7 +43,6 @@ namespace {
 
 constexpr int kMaxSplitsF = 64;
 constexpr int kRowsP = 64;               // query rows per prefill workgroup, 16 per wave
-constexpr unsigned kGroupWgs = 1024;     // prefill calls of up to this many workgroups take two key groups each
 constexpr int kRunP = 128;               // prefill: keys per run are a multiple of this
 
 constexpr int kWavesD = 4;               // decode: waves per workgroup, a 16-key tile each at a time
@@ -357,12 +356,9 @@ __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args 
   const int r = lane & 15, gq = lane >> 4;
   // Slots of one tile position follow each other over (KV head, run), the last tiles
   // (most keys) first; empty slots of the grid's upper bound before them.
-  const int64_t work = (int64_t)p.row_tiles * p.num_kv_heads * p.splits;
-  if ((int64_t)blockIdx.x >= work) {  // a padded grid's pad rows: one workgroup per sequence
-    zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, (int)(blockIdx.x - work), p.out, p.out_stride,
-                  (int64_t)p.num_qo_heads * D, (int64_t)p.batch * p.grid_width);
-    return;
-  }
+  if (p.q_rows)
+    zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, p.batch, p.out, p.out_stride * 4, p.num_qo_heads * D * 4,
+                  blockIdx.x * (kThreads / 64) + (tid >> 6), gridDim.x * (kThreads / 64));
   const int runs = p.num_kv_heads * p.splits;
   const int run = blockIdx.x % runs;
   const int split = run / p.num_kv_heads, h = run - split * p.num_kv_heads;  // a head's runs on one XCD
@@ -621,7 +617,12 @@ void launch_merge_f32(const AttnF32Args& p, hipStream_t s) {
 template <int D>
 int launch_f32(const AttnF32Args& p, dim3 grid, hipStream_t s) {
   if (p.qo_indptr) {
-    if (grid.x <= kGroupWgs)
+    // Two groups of waves on each row tile, half of an LDS tile's keys each, where one group
+    // leaves SIMDs idle: fresh prompts of few tiles (4 x 128 tokens 25.5 -> 24.0 us, 4 x
+    // 100..512 47.6 -> 42.4; D = 64, 4 x 512, 105 -> 84). Not for calls of many workgroups
+    // (8 x 512 over 512: 542 us, with two groups 646), calls cut into runs (512 from zero
+    // 57.3 and 63.5), nor a few short tiles (16 tokens 10.9 and 12.5).
+    if (p.splits == 1 && grid.x > 32 && grid.x <= (D == 64 ? 2048u : 1024u))
       prefill_f32_kernel<D, 2><<<grid, 512, 0, s>>>(p);
     else
       prefill_f32_kernel<D, 1><<<grid, 256, 0, s>>>(p);
@@ -687,8 +688,8 @@ int attention_f32(const AttnF32Args& a, int32_t head_dim, hipStream_t s) {
     // row-tile slots per (KV head, run): an upper bound over the batch (every sequence
     // may end in a partial tile)
     const int64_t tiles = (a.total_q * a.group + kRowsP - 1) / kRowsP + a.batch;
-    const int64_t wgs = tiles * a.num_kv_heads * a.splits + (a.q_rows ? a.batch : 0);
-    if (wgs > 0x7fffffff) return fail(NSLG_EUNSUPPORTED, "attention_f32: too many rows");
+    const int64_t wgs = tiles * a.num_kv_heads * a.splits;
+    if (wgs > 0x7fffffff / 8) return fail(NSLG_EUNSUPPORTED, "attention_f32: too many rows");
     p.row_tiles = (int32_t)tiles;
     grid = dim3((unsigned)wgs);
   } else {

@@ -164,28 +164,28 @@ __device__ inline void stream_store(V* p, V v) {
 }
 
 // ---- padded output grids of the prefill entries ----------------------------------
-// One workgroup's share of a padded grid of batch x width rows (row_elems elements
-// each, rows 16-byte aligned): the rows of sequence b's block (rows b * width ..
-// b * width + width - 1) that hold none of its new tokens are set to zero. The
-// sequence's n_b = qo[b + 1] - qo[b] tokens sit at rows q_rows[qo[b]] .. + n_b - 1,
-// contiguous and inside the block (the forward's padded layout).
-template <typename E>
-__device__ inline void zero_pad_rows(const int32_t* qo, const int32_t* q_rows, int width, int b, E* out,
-                                     int64_t out_stride, int64_t row_elems, int64_t grid_rows) {
-  const int q0 = qo[b];
-  const int n = qo[b + 1] - q0;
-  int64_t first = n > 0 ? (int64_t)q_rows[q0] - (int64_t)b * width : 0;
-  first = first < 0 ? 0 : (first > width ? width : first);
-  int64_t last = first + (n > 0 ? n : 0);
-  last = last > width ? width : last;
-  const int64_t vecs = row_elems * (int64_t)sizeof(E) / 16;
-  const int64_t pads = width - (last - first);
+// A wave's share of a padded grid of batch x width rows (row_bytes each, a multiple of
+// 16, 16-byte aligned): of rows first, first + step, ..., those that hold no new token
+// are set to zero. Sequence b's n_b = qo[b + 1] - qo[b] tokens sit at rows q_rows[qo[b]]
+// .. + n_b - 1, contiguous and inside its block of `width` rows (the forward's padded
+// layout). Every wave of the launch takes a share: the pads are up to half of the
+// output, and one workgroup per sequence took longer to zero them (2.5 MB for 156 rows
+// of 16 KB, 100 us) than the others to attend (prompts of 128 to 284 tokens, 30 us).
+inline __device__ void zero_pad_rows(const int32_t* qo, const int32_t* q_rows, int width, int batch, void* out,
+                                     int64_t out_row_bytes, int row_bytes, int first, int step) {
+  const int lane = threadIdx.x & 63;
+  const int rows = batch * width;  // < 2^31 (checked by the host)
   const u32x4 z = {0u, 0u, 0u, 0u};
-  for (int64_t i = threadIdx.x; i < pads * vecs; i += blockDim.x) {
-    const int64_t pr = i / vecs;
-    const int64_t r = (int64_t)b * width + (pr < first ? pr : pr + (last - first));
-    if (r >= grid_rows) continue;
-    *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(out + r * out_stride) + 16 * (i - pr * vecs)) = z;
+  for (int64_t at_row = __builtin_amdgcn_readfirstlane(first); at_row < rows; at_row += step) {
+    const int r = (int)at_row, b = r / width, c = r - b * width;
+    const int q0 = qo[b], n = qo[b + 1] - q0;
+    if (n > 0) {
+      const int64_t at = (int64_t)q_rows[q0] - (int64_t)b * width;
+      const int64_t lo = at < 0 ? 0 : at;
+      if (c >= lo && c < lo + n) continue;  // a token's row
+    }
+    char* row = static_cast<char*>(out) + (int64_t)r * out_row_bytes;
+    for (int i = 16 * lane; i < row_bytes; i += 1024) *reinterpret_cast<u32x4*>(row + i) = z;
   }
 }
 

@@ -87,14 +87,12 @@ struct PrefillParams {
   int64_t out_stride;
   int32_t row_tiles;  // row-tile slots per KV head (an upper bound over the batch)
   int32_t num_work;   // row_tiles * num_kv_heads
-  int32_t per_xcd;    // ceil((num_work + pad_work) / 8)
+  int32_t per_xcd;    // ceil(num_work / 8)
   // Grid rows (null: q and out are the ragged rows themselves): ragged row t is row
   // q_rows[t] of q and out, [batch x grid_width] rows, sequence b's block being rows
-  // b * grid_width .. + grid_width - 1; pad_work workgroups zero the rows of each
-  // block that hold no new token.
+  // b * grid_width .. + grid_width - 1; the rows that hold no new token are set to zero.
   const int32_t* q_rows;
   int32_t grid_width;
-  int32_t pad_work;
   int32_t by_round;   // > 0: longest-first rounds of this many tiles per sequence (see below)
   int32_t rows_wg;    // query rows per workgroup (the kernel's tile shape)
   // The forward's new K/V rows (k_new null: already in the pool). Token t of sequence
@@ -246,12 +244,10 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   // last. Between the full ones they keep CUs from work: a tile of 17 runs, every other
   // slot empty, took 35 us, of 9 runs 13 us (16 of an XCD's CUs got the full slots).
   const int w = kSplit ? (int)blockIdx.x : (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
-  if (w >= p.num_work) {
-    if (w < p.num_work + p.pad_work)
-      zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, w - p.num_work, p.out, p.out_stride,
-                    (int64_t)p.num_qo_heads * D, (int64_t)p.batch * p.grid_width);
-    return;
-  }
+  if (w >= p.num_work) return;
+  if (p.q_rows)
+    zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, p.batch, p.out, p.out_stride * 2, p.num_qo_heads * D * 2,
+                  w * kWaves + wave, p.num_work * kWaves);
   const int runs = p.num_kv_heads * p.splits;
   const int run = kSplit ? w % runs : w / p.row_tiles;  // (KV head, run of keys)
   const int h = kSplit ? run % p.num_kv_heads : run;
@@ -1032,9 +1028,8 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
   p.num_work = (int32_t)(slots * num_kv_heads * p.splits);
   p.q_rows = q_rows;
   p.grid_width = grid_width;
-  p.pad_work = q_rows ? batch : 0;
-  if ((int64_t)p.num_work + p.pad_work > 0x7fffffff - 8) return fail(NSLG_EUNSUPPORTED, "paged_prefill: too many rows");
-  p.per_xcd = (p.num_work + p.pad_work + 7) / 8;
+  if ((int64_t)p.num_work > 0x7fffffff / 8 - 8) return fail(NSLG_EUNSUPPORTED, "paged_prefill: too many rows");
+  p.per_xcd = (p.num_work + 7) / 8;
   p.k_new = (const uint16_t*)k_new;
   p.v_new = (const uint16_t*)v_new;
   p.k_new_stride = k_new_stride;

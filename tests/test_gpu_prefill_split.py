@@ -70,3 +70,33 @@ def test_prefill_in_runs_writes_the_new_rows(dtype, D, grid):
     o2 = K.paged_prefill(q, d(qo), sum(news), max(news), k2, v2, *plan, **kw)
     torch.cuda.synchronize()
     assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(o1, o2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 128), (torch.bfloat16, 256), (torch.float32, 64)])
+@pytest.mark.parametrize("news,W", [([1, 0, 700], 700), ([3], 2500), ([0, 0], 9)])
+def test_pad_rows_shared_by_the_launch(news, W, dtype, D):
+    """Padded grids of mostly pad rows (more of them than the launch has waves, a sequence
+    without tokens, no token at all): pad rows zero, token rows those of the ragged call."""
+    from nanoslg_amd import kernels as K
+    Hq, Hkv, ps, B = 8, 2, 16, len(news)
+    g = torch.Generator().manual_seed(W)
+    npg = [-(-n // ps) for n in news]
+    qo = np.concatenate([[0], np.cumsum(news)]).astype(np.int32)
+    indptr = np.concatenate([[0], np.cumsum(npg)]).astype(np.int32)
+    ids = np.arange(1, sum(npg) + 1, dtype=np.int32) if sum(npg) else np.zeros(1, np.int32)
+    lpl = np.array([(n - 1) % ps + 1 if n else 0 for n in news], np.int32)
+    rows = np.concatenate([b * W + W - n + np.arange(n) for b, n in enumerate(news)] + [np.zeros(1)]).astype(np.int32)
+    k, v = (torch.randn(sum(npg) + 1, ps, Hkv, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+    q = torch.randn(B * W, Hq, D, generator=g).to(dtype).to(DEV)
+    d = lambda a: torch.from_numpy(a).to(DEV)  # noqa: E731
+    plan = (k, v, d(indptr), d(ids), d(lpl))
+    T = sum(news)
+    out = torch.full_like(q, 7.0)
+    K.paged_prefill(q, d(qo), T, max(news), *plan, out=out, q_rows=d(rows), grid_width=W)
+    at = torch.from_numpy(rows[:T].astype(np.int64)).to(DEV)
+    want = torch.zeros_like(q)
+    if T:
+        want[at] = K.paged_prefill(q[at].contiguous(), d(qo), T, max(news), *plan)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
