@@ -343,9 +343,9 @@ int nslg_paged_decode_grouped_rope_append(
  *               [qo_indptr[b], qo_indptr[b+1]) and sit at the LAST positions of
  *               that sequence's L_b tokens (bottom-right causal alignment):
  *               row t of b attends to keys j <= L_b - n_b + t.
- *   total_q     host copy of qo_indptr[batch]; max_q: host max of n_b (sizes the
- *               longest-first tile order of near-uniform batches; a value below
- *               the true max only costs that order, never correctness)
+ *   total_q     host copy of qo_indptr[batch]; max_q: host max of n_b (sizes the runs
+ *               that the keys of a call of few row tiles are cut into; a wrong value
+ *               only costs time, never correctness)
  *   out         [T] rows of Hq*D elements at stride out_stride
  *   sm_scale    positive and finite (EINVAL otherwise)
  *   workspace   of nslg_paged_prefill_workspace_size bytes, not shared with a call

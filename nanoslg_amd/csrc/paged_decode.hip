@@ -130,17 +130,6 @@ __device__ inline int seq_len_of(const int32_t* indptr, const int32_t* last_len,
   return (np - 1) * page_size + lpl;
 }
 
-__device__ inline int wave_sum_i32(int x) {
-  x += __builtin_amdgcn_mov_dpp(x, 0x128, 0xf, 0xf, false);  // row_ror:8
-  x += __builtin_amdgcn_mov_dpp(x, 0x124, 0xf, 0xf, false);  // row_ror:4
-  x += __builtin_amdgcn_mov_dpp(x, 0x122, 0xf, 0xf, false);  // row_ror:2
-  x += __builtin_amdgcn_mov_dpp(x, 0x121, 0xf, 0xf, false);  // row_ror:1
-  const auto a = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)x, false, false);
-  x = (int)(a[0] + a[1]);
-  const auto c = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)x, false, false);
-  return (int)(c[0] + c[1]);
-}
-
 // Tokens of the prefix of group g (its first member's length bounds it, so the
 // prefix never reads past that member's block table).
 __device__ inline int group_prefix_tokens(const DecodeParams& p, const GroupArgs<true>& ga, int g) {

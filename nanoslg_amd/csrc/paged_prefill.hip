@@ -85,16 +85,12 @@ struct PrefillParams {
   float scale_log2;
   uint16_t* out;
   int64_t out_stride;
-  int32_t row_tiles;  // row-tile slots per KV head (an upper bound over the batch)
-  int32_t num_work;   // row_tiles * num_kv_heads
-  int32_t per_xcd;    // ceil(num_work / 8)
+  int32_t num_work;   // row-tile slots (an upper bound over the batch) x KV heads x runs
   // Grid rows (null: q and out are the ragged rows themselves): ragged row t is row
   // q_rows[t] of q and out, [batch x grid_width] rows, sequence b's block being rows
   // b * grid_width .. + grid_width - 1; the rows that hold no new token are set to zero.
   const int32_t* q_rows;
   int32_t grid_width;
-  int32_t by_round;   // > 0: longest-first rounds of this many tiles per sequence (see below)
-  int32_t rows_wg;    // query rows per workgroup (the kernel's tile shape)
   // The forward's new K/V rows (k_new null: already in the pool). Token t of sequence
   // b is row r_b + t of k_new / v_new, r_b the row of its first token (q's row map);
   // keys at positions >= start_b are read from these rows, and the workgroup holding
@@ -138,76 +134,6 @@ __device__ inline int64_t grid_row(const PrefillParams& p, int t) {
   return r >= 0 && r < (int64_t)p.batch * p.grid_width ? r : -1;
 }
 
-__device__ inline int kv_len_of(const PrefillParams& p, int s) {
-  const int np = p.indptr[s + 1] - p.indptr[s];
-  if (np <= 0) return 0;
-  int lpl = p.last_len[s];
-  lpl = lpl < 1 ? 1 : (lpl > p.page_size ? p.page_size : lpl);
-  return (np - 1) * p.page_size + lpl;
-}
-
-// Longest first: slot g is round r = g / batch of sequence g % batch, and round r
-// takes each sequence's r-th tile from the end. A later row tile sees more keys
-// (causal), so the first slots dispatched carry the most work and the short tiles
-// fill in behind them. Slots past a sequence's tiles are empty.
-__device__ inline bool locate_tile_by_round(const PrefillParams& p, int g, int& b, int& tile) {
-  b = g % p.batch;
-  const int r = g / p.batch;
-  const int n = p.qo_indptr[b + 1] - p.qo_indptr[b];
-  const int nt = n > 0 ? (n * p.group + p.rows_wg - 1) / p.rows_wg : 0;
-  if (r >= nt) return false;
-  tile = nt - 1 - r;
-  return true;
-}
-
-// Most row tiles of any sequence of the batch (wave-wide, uniform).
-__device__ inline int most_tiles(const PrefillParams& p) {
-  const int lane = threadIdx.x & 63;
-  int most = 0;
-  for (int s0 = 0; s0 < p.batch; s0 += 64) {
-    const int s = s0 + lane;
-    int nt = 0;
-    if (s < p.batch) {
-      const int n = p.qo_indptr[s + 1] - p.qo_indptr[s];
-      nt = n > 0 ? (n * p.group + p.rows_wg - 1) / p.rows_wg : 0;
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) nt = max(nt, __shfl_xor(nt, off, 64));
-    most = max(most, nt);
-  }
-  return __builtin_amdgcn_readfirstlane(most);
-}
-
-// Wave-wide search for the (sequence, row tile) of workgroup x.
-__device__ inline bool locate_tile(const PrefillParams& p, int g, int& b, int& tile) {
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  for (int s0 = 0; s0 < p.batch; s0 += 64) {
-    const int s = s0 + lane;
-    int nt = 0;
-    if (s < p.batch) {
-      const int n = p.qo_indptr[s + 1] - p.qo_indptr[s];
-      nt = n > 0 ? (n * p.group + p.rows_wg - 1) / p.rows_wg : 0;
-    }
-    int incl = nt;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int y = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += y;
-    }
-    const int excl = incl - nt;
-    const unsigned long long m = __ballot(nt > 0 && g >= base + excl && g < base + incl);
-    if (m) {
-      const int src = __ffsll((long long)m) - 1;
-      b = s0 + src;
-      tile = g - base - __shfl(excl, src, 64);
-      return true;
-    }
-    base += __shfl(incl, 63, 64);
-  }
-  return false;
-}
-
 template <typename T, int D, bool kSplit>
 __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_kernel(PrefillParams p) {
   constexpr int kCB = PrefillTile<D>::kCB;
@@ -236,34 +162,23 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  // XCD-aware order: workgroup i runs on XCD i % 8, so work item
-  // w = (i % 8) * per_xcd + i / 8 gives each XCD a contiguous run of row tiles of
-  // one KV head, which read the same K/V and so share that XCD's L2.
-  // kSplit: work item = workgroup, the tiles' first slots before the last ones and the
-  // (KV head, run) pairs in turn: the empty slots of the grid's upper bound then come
-  // last. Between the full ones they keep CUs from work: a tile of 17 runs, every other
-  // slot empty, took 35 us, of 9 runs 13 us (16 of an XCD's CUs got the full slots).
-  const int w = kSplit ? (int)blockIdx.x : (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
+  // Work item = workgroup: the tile's slot (longest first), then (run of keys, KV head) in
+  // turn. Workgroup i runs on XCD i % 8, so with 8 KV heads an XCD has one head, all its
+  // row tiles and runs, which read the same K/V and so share its L2; the empty slots of
+  // the grid's upper bound come last (between the full ones they kept CUs from work: a
+  // tile of 17 runs, every other slot empty, took 35 us, of 9 runs 13 us).
+  const int w = (int)blockIdx.x;
   if (w >= p.num_work) return;
   if (p.q_rows)
     zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, p.batch, p.out, p.out_stride * 2, p.num_qo_heads * D * 2,
                   w * kWaves + wave, p.num_work * kWaves);
-  const int runs = p.num_kv_heads * p.splits;
-  const int run = kSplit ? w % runs : w / p.row_tiles;  // (KV head, run of keys)
+  const int runs = kSplit ? p.num_kv_heads * p.splits : p.num_kv_heads;
+  const int run = w % runs;
   const int h = kSplit ? run % p.num_kv_heads : run;
-  int b = 0, tile = 0;
-  const int g = kSplit ? w / runs : w - run * p.row_tiles;
-  // longest-first rounds when the host's round count covers every sequence (it came
-  // from the caller's max_q); otherwise the packed order, which the grid also fits
-  const bool rounds = p.by_round > 0 && most_tiles(p) <= p.by_round;
-  if (!(rounds ? locate_tile_by_round(p, g, b, tile) : locate_tile(p, g, b, tile)))
+  PrefillSeq sq;
+  if (!locate_row_tile(p.qo_indptr, p.indptr, p.last_len, p.page_size, p.batch, p.group, kRowsPerWG, w / runs, sq))
     return;  // uniform across the workgroup
-  b = __builtin_amdgcn_readfirstlane(b);
-  tile = __builtin_amdgcn_readfirstlane(tile);
-
-  const int q0 = p.qo_indptr[b];
-  const int n_new = p.qo_indptr[b + 1] - q0;
-  const int L = kv_len_of(p, b);
+  const int b = sq.b, tile = sq.tile, q0 = sq.q0, n_new = sq.n_new, L = sq.len;
   const int start = L - n_new > 0 ? L - n_new : 0;  // position of the first new token
   const int G = p.group;
   const int nrows = n_new * G;
@@ -273,6 +188,7 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   const int kv_end = min(L, start + last_row / G + 1);
   int kt_first = 0;
   int n_kt = (kv_end + kKeys - 1) / kKeys;
+  bool merged = false;  // the tile's keys are in more than one run
   int parts = 1;
   if constexpr (kSplit) {
     // equal runs of key tiles, of at least kMinRun tiles each
@@ -280,6 +196,7 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
     const int per = max((n_kt + p.splits - 1) / p.splits, kMinRun);
     parts = max((n_kt + per - 1) / per, 1);
     if (split >= parts) return;
+    merged = parts > 1;
     kt_first = split * per;
     n_kt = min(n_kt, kt_first + per);
   }
@@ -326,6 +243,10 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
     const int t = row_ok[cb] ? row / G : 0;
     row_tok[cb] = start + t;  // absolute position of this row's token
     const int64_t qr = row_ok[cb] ? grid_row(p, q0 + t) : -1;
+    if constexpr (kSplit) {
+      if (kt_first == 0 && gq == 0 && row_ok[cb] && q0 + t < p.total_q)
+        p.part_count[(int64_t)(q0 + t) * p.num_qo_heads + h * G + row % G] = parts;
+    }
     if (qr >= 0) {
       const uint16_t* qrow = p.q + qr * p.q_stride + (int64_t)(h * G + row % G) * D;
 #pragma unroll
@@ -342,21 +263,20 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   // lowest position among the wave's rows: keys below start + first_tok + 1 are visible to all
   const int wave_first_tok = __builtin_amdgcn_readfirstlane(start + (row0_wg + wave * kRowsPerWave) / G);
 
-  float m_run[kCB];
   // row sums of P on the MFMA: an all-ones A operand makes every row of the 16x16
   // output tile the column's sum over the block's keys
   f32x4 lsum[kCB];
   const unsigned short one16 = T::from_f32(1.f);
   const u16x8 ones = u16x8{one16, one16, one16, one16, one16, one16, one16, one16};
   // per column block: raw-score threshold above which the running max must be raised,
-  // and the exponent offset -m (0 while m = -inf); both change only with m
+  // and the exponent offset -m (0 while m = -inf); both change only with m, which is not
+  // held itself (two registers that the block loop has not got)
   float thr[kCB];
   float neg_m[kCB];
   const float inv_scale_log2 = 1.f / p.scale_log2;
   f32x4 o[kCB][NT];
 #pragma unroll
   for (int cb = 0; cb < kCB; ++cb) {
-    m_run[cb] = -INFINITY;
     thr[cb] = -INFINITY;
     neg_m[cb] = 0.f;
     lsum[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -531,6 +451,7 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
       va[n] = __builtin_bit_cast(u16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
   };
+  auto run_max = [&](int cb) { return thr[cb] == -INFINITY ? -INFINITY : -neg_m[cb]; };
   // masking (blocks touching the causal diagonal or the end of the keys) and the lazy
   // rescale: the row's running max m is raised only when some score of the block
   // exceeds it by more than the slack, which each lane checks on its own 8 scores;
@@ -550,12 +471,12 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
       const float lmax = fmaxf(fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3])),
                                fmaxf(fmaxf(b[0], b[1]), fmaxf(b[2], b[3])));
       if (__ballot(lmax > thr[cb])) {
-        const float m_new = fmaxf(m_run[cb], rows_max(lmax * p.scale_log2));
-        const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run[cb] - m_new);
+        const float m_run = run_max(cb);
+        const float m_new = fmaxf(m_run, rows_max(lmax * p.scale_log2));
+        const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(m_run - m_new);
         lsum[cb] *= alpha;
 #pragma unroll
         for (int n = 0; n < NT; ++n) o[cb][n] *= alpha;
-        m_run[cb] = m_new;
         thr[cb] = (m_new + kRescaleSlack) * inv_scale_log2;
         neg_m[cb] = m_new == -INFINITY ? 0.f : -m_new;
       }
@@ -748,10 +669,9 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
     if constexpr (kSplit) {
       const int64_t pr = (int64_t)(q0 + t) * p.num_qo_heads + h * G + row % G;
       if (q0 + t >= p.total_q) continue;  // past the partials: not a row of this call
-      if (kt_first == 0 && gq == 0) p.part_count[pr] = parts;
-      if (parts > 1) {
+      if (merged) {
         const int64_t slot = (int64_t)(run / p.num_kv_heads) * p.total_q * p.num_qo_heads + pr;
-        if (gq == 0) p.part_ml[slot] = float2{m_run[cb], l_tot};
+        if (gq == 0) p.part_ml[slot] = float2{run_max(cb), l_tot};
         float* po = p.part_o + slot * D + 4 * gq;
 #pragma unroll
         for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4*>(po + 16 * n) = o[cb][n];
@@ -838,7 +758,7 @@ template <typename T, int D>
 int launch_prefill(const PrefillParams& p, hipStream_t s) {
   // D = 64, 128: two column blocks (32 rows) per wave, 8 waves: measured faster than
   // four per wave at one wave per SIMD (chunk 3584..4095 of 8 x 4096: 276 vs 338 us)
-  const dim3 grid((unsigned)(8 * p.per_xcd));
+  const dim3 grid((unsigned)p.num_work);
   constexpr int kThreads = 64 * PrefillTile<D>::kWaves;
   if (p.splits == 1) {
     paged_prefill_kernel<T, D, false><<<grid, kThreads, 0, s>>>(p);
@@ -993,19 +913,7 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   p.out = (uint16_t*)out;
   p.out_stride = out_stride;
-  if (tiles * num_kv_heads > 0x7fffffff) return fail(NSLG_EUNSUPPORTED, "paged_prefill: too many rows");
-  // Longest-first rounds need batch x (most tiles of a sequence) slots; taken when
-  // that is at most 5/4 of the slots of the packed order (near-uniform batches,
-  // such as the chunks of a batch of prompts), so few slots are empty.
-  // The grid fits both orders; the kernel checks the rounds against the batch.
-  const int64_t most = max_q > 0 ? ((int64_t)max_q * group + rows_wg - 1) / rows_wg : 0;
-  const int64_t round_slots = (int64_t)batch * most;
-  const bool by_round = most > 0 && most <= 0x7fffffff && 4 * round_slots <= 5 * tiles;
-  p.by_round = by_round ? (int32_t)most : 0;
-  p.rows_wg = rows_wg;
-  const int64_t slots = by_round && round_slots > tiles ? round_slots : tiles;
-  if (slots * num_kv_heads > 0x7fffffff) return fail(NSLG_EUNSUPPORTED, "paged_prefill: too many rows");
-  p.row_tiles = (int32_t)slots;
+  if (tiles * num_kv_heads * kMaxSplits > 0x7fffffff) return fail(NSLG_EUNSUPPORTED, "paged_prefill: too many rows");
   p.total_q = total_q;
   p.splits = 1;
   p.part_o = nullptr;
@@ -1025,11 +933,9 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
       p.part_o = (float*)ws;
     }
   }
-  p.num_work = (int32_t)(slots * num_kv_heads * p.splits);
+  p.num_work = (int32_t)(tiles * num_kv_heads * p.splits);
   p.q_rows = q_rows;
   p.grid_width = grid_width;
-  if ((int64_t)p.num_work > 0x7fffffff / 8 - 8) return fail(NSLG_EUNSUPPORTED, "paged_prefill: too many rows");
-  p.per_xcd = (p.num_work + 7) / 8;
   p.k_new = (const uint16_t*)k_new;
   p.v_new = (const uint16_t*)v_new;
   p.k_new_stride = k_new_stride;
