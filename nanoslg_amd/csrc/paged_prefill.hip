@@ -776,9 +776,15 @@ int launch_prefill(const PrefillParams& p, hipStream_t s) {
 // half kCUs workgroups leaves CUs idle for as long as one workgroup walks its keys: its
 // tiles' keys are cut so that the workgroups fill the CUs once.
 int prefill_splits(int64_t total_q, int32_t batch, int32_t max_q, int group, int32_t num_kv_heads, int rows_wg) {
-  int64_t tiles = (total_q * group + rows_wg - 1) / rows_wg;  // at least this many
-  if (max_q > 0 && (int64_t)max_q * batch == total_q)         // a uniform batch: exactly
+  int64_t tiles;
+  if (max_q > 0 && (int64_t)max_q * batch == total_q) {  // a uniform batch
     tiles = batch * (((int64_t)max_q * group + rows_wg - 1) / rows_wg);
+  } else {
+    // a ragged one ends each sequence in a tile half full on average, and has one each at
+    // least (without these, 13 short suffixes were cut into 10 runs each: 114 -> 133 us)
+    tiles = (total_q * group + rows_wg - 1) / rows_wg + batch / 2;
+    tiles = tiles > batch ? tiles : batch;
+  }
   const int64_t wgs = tiles * num_kv_heads;
   const int64_t s = kCUs / (wgs < 1 ? 1 : wgs);
   return (int)(s < 1 ? 1 : (s > kMaxSplits ? kMaxSplits : s));

@@ -181,11 +181,10 @@ def rope_append(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, posit
     if q_out.shape != q.shape or q_out.dtype != q.dtype:
         raise ValueError("rope_append: q_out must be shaped like q")
     no, qos, _ = _rows(q_out, "q_out")
-    rc = _lib.load().nslg_rope_append(q.data_ptr(), qs, q_out.data_ptr(), qos, k_new.data_ptr(), ks,
-                                      v_new.data_ptr(), vs, positions.data_ptr(), slot_mapping.data_ptr(), T,
-                                      cos.data_ptr(), sin.data_ptr(), cos.stride(0), cos.shape[0], Hq, Hkv, D,
-                                      k_pool.data_ptr(), v_pool.data_ptr(), k_pool.numel() // (Hkv * D),
-                                      dtype_code(q.dtype), _stream(q))
+    rc = _lib.fast().rope_append(q.data_ptr(), qs, q_out.data_ptr(), qos, k_new.data_ptr(), ks, v_new.data_ptr(), vs,
+                                 positions.data_ptr(), slot_mapping.data_ptr(), T, cos.data_ptr(), sin.data_ptr(),
+                                 cos.stride(0), cos.shape[0], Hq, Hkv, D, k_pool.data_ptr(), v_pool.data_ptr(),
+                                 k_pool.numel() // (Hkv * D), dtype_code(q.dtype), _stream(q))
     _lib.check(rc, "nslg_rope_append")
     return q_out
 
@@ -891,10 +890,12 @@ _PREFILL_WS: Dict[Tuple[int, int, int, int, int], int] = {}  # nslg_paged_prefil
 
 
 # Keys of the longest sequence from which a prefill call gets a workspace, so that the
-# library may cut its row tiles' keys into runs. Measured at 32/8 heads x 128, one
-# sequence: 512 new tokens from zero 25.7 us either way (bf16 31.1 -> 27.5), 256 from
-# zero 17.7 us in one run and 20.4 in runs, 16 over 512 18.8 and 14.4.
-PREFILL_SPLIT_KEYS = 512
+# library may cut its row tiles' keys into runs (by head dim: a tile of 64-wide keys is
+# over in half the time). Runs cost a merge launch, an allocation and a pass over the
+# partials, about 8 us of a call: measured at 32/8 heads, 7 x 21 tokens over 588 keys 45
+# us and 47 in runs, 6 x 64..99 over 417 at D = 64 35 and 42, 2 x 121 over 1117 62 and 34,
+# and over 45 draws of larger contexts 2.3 times as fast (geometric mean).
+PREFILL_SPLIT_KEYS = {64: 1024, 128: 768, 256: 768}
 
 
 def _prefill_workspace(q, B, Hq, D, total_q, max_q, max_kv):
@@ -902,7 +903,7 @@ def _prefill_workspace(q, B, Hq, D, total_q, max_q, max_kv):
     max_kv keys; (None, None, 0) where the call takes its keys in one run. From the caching
     allocator on the current stream, and not the cache's workspace: one cache's prefills
     may run on another stream than its decodes."""
-    if max_kv < PREFILL_SPLIT_KEYS:
+    if max_kv < PREFILL_SPLIT_KEYS.get(D, 1 << 62):
         return None, None, 0
     key = (B, Hq, D, total_q, max_q)
     need = _PREFILL_WS.get(key)

@@ -1823,6 +1823,7 @@ class ContiguousCacheContext(CacheContext):
         pos, q_rows, qo = _ragged_layout(self.start_positions, self.new_token_counts, self.input_offsets, iw)
         self._max_q = max(self.new_token_counts) if B else 0
         self._uniform_rows = int(qo[-1]) == B * iw
+        self._decode_launch = None
         self._plan = _ForwardPlan(cache.device, B, iw, slot.reshape(-1), pos, indptr, indices, lpl, qo,
                                   q_rows, np.zeros(0, np.int32), np.zeros(0, np.int32))
 
@@ -1834,8 +1835,10 @@ class ContiguousCacheContext(CacheContext):
 
     def attend(self, layer_idx, q, k_new, v_new, n_heads, n_kv_heads):
         cache, plan = self.cache, self._plan
-        k_layer, v_layer = cache.paged_view(layer_idx)
         B, S = q.shape[0], q.shape[1]
+        if self._in_one_launch(S, q, k_new, v_new):
+            return self._decode(q)(layer_idx % cache.cfg.num_layers, q, k_new, v_new)
+        k_layer, v_layer = cache.paged_view(layer_idx)
         if not (self._is_decode and S == 1):
             # the write and the attention in one launch (a sequence's slot is its one page)
             uniform = self._uniform_rows and S == self._iw
@@ -1859,10 +1862,40 @@ class ContiguousCacheContext(CacheContext):
         if self.max_kv_len > cos.shape[0]:
             raise IndexError(f"position {self.max_kv_len - 1} is outside the rope tables ({cos.shape[0]} rows)")
         S = q.shape[1]
+        if self._in_one_launch(S, q, k_new, v_new):
+            return self._decode(q)(layer_idx % cache.cfg.num_layers, q, k_new, v_new,
+                                   rope=(cos, sin, plan.pos_for(S)))
         k_layer, v_layer = cache.paged_view(layer_idx)
         q_rot = cache.kernels.rope_append(q, k_new, v_new, plan.pos_for(S), plan.slots_for(S), cos, sin,
                                           k_layer, v_layer)
         return self._attend_written(q_rot, k_layer, v_layer)
+
+    def _in_one_launch(self, S, q, k_new, v_new):
+        """A decode step whose rows the decode launch writes itself (a padded step's row,
+        and tensors of another type, take the separate calls)."""
+        return (self._is_decode and S == 1 and self._iw == 1
+                and q.dtype == k_new.dtype == v_new.dtype == self.cache.cfg.dtype)
+
+    def _decode(self, q):
+        """The forward's decode launcher (kernels.DecodeLaunch) over the slots, each a page
+        of max_seq_len tokens; the previous forward's, re-bound, when batch and heads stay."""
+        cache, plan = self.cache, self._plan
+        launch = self._decode_launch
+        if launch is None:
+            launch, kern = cache._launcher, cache.kernels
+            if (launch is not None and hasattr(launch, "rebind") and launch.B == plan.batch
+                    and launch.Hq == q.shape[2] and launch.pools[0] is cache.k and launch.pools[1] is cache.v):
+                launch.rebind(plan.slot, plan.indptr, plan.indices, plan.lpl, plan.total_pages, check=False)
+            else:
+                launch = cache._launcher = kern.DecodeLaunch(cache.k, cache.v, plan.slot, plan.indptr, plan.indices,
+                                                             plan.lpl, plan.total_pages, q.shape[2],
+                                                             workspace=cache.workspace)
+            launch.bound_plan = plan
+            self._decode_launch = launch
+        elif launch.bound_plan is not plan:  # another forward was begun since
+            launch.rebind(plan.slot, plan.indptr, plan.indices, plan.lpl, plan.total_pages, check=False)
+            launch.bound_plan = plan
+        return launch
 
     def _attend_written(self, q, k_layer, v_layer):
         """Attention of the forward's rows over the slots (K/V already written)."""
@@ -1898,6 +1931,7 @@ class ContiguousKVCache(KVCacheManager):
         self.states: Dict[str, _ContigSeqState] = {}
         self._slot = 0
         self.workspace = self.kernels.Workspace(self.device, 16 << 20)
+        self._launcher = None  # the last decode forward's kernels.DecodeLaunch
 
     def paged_view(self, layer_idx):
         return self.k[layer_idx], self.v[layer_idx]

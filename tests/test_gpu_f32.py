@@ -60,3 +60,45 @@ def test_f32_decode_writes_the_new_rows(D):
     o2 = K.paged_decode(q, k2, v2, *plan)
     torch.cuda.synchronize()
     assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(o1, o2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_contiguous_decode_in_one_launch(dtype):
+    """Decode steps of the contiguous cache against append_kv then paged_decode on a copy:
+    pool bytes and outputs equal; two contexts of different batches alive at once, a
+    negative layer index, rows off 16 bytes and a changed batch included."""
+    from nanoslg_amd import kernels as K
+    from nanoslg_amd.kv_cache import ContiguousKVCache, KVCacheConfig
+    L, Hq, Hkv, D, Smax = 2, 8, 2, 64, 77
+    m = ContiguousKVCache(KVCacheConfig(num_layers=L, num_kv_heads=Hkv, num_qo_heads=Hq, head_dim=D, max_batch_size=3,
+                                        max_seq_len=Smax, dtype=dtype, device=torch.device(DEV), backend="contiguous"))
+    g = torch.Generator().manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)  # noqa: E731
+    ids = ["a", "b", "c"]
+    for s in ids:
+        m.allocate_sequence(s)
+    ctx = m.begin_forward(ids, [40, 3, 75])
+    for layer in range(L):
+        ctx.attend(layer, rnd(3, 75, Hq, D), rnd(3, 75, Hkv, D), rnd(3, 75, Hkv, D), Hq, Hkv)
+    m.end_forward(ctx)
+
+    def step(ctx, batch, layer):
+        B, plan = len(batch), ctx._plan
+        q, rows = rnd(B, 1, Hq, D), rnd(2, B, Hkv * D + 1)
+        k, v = (x[:, 1:].reshape(B, 1, Hkv, D) if layer else x[:, 1:].unflatten(1, (Hkv, D)).unsqueeze(1) for x in rows)
+        kc, vc = m.k[layer].clone(), m.v[layer].clone()
+        out = ctx.attend(layer, q, k, v, Hq, Hkv)
+        K.append_kv(k, v, plan.slot, kc, vc)
+        want = K.paged_decode(q[:, 0], kc, vc, plan.indptr, plan.indices, plan.lpl, plan.total_pages)
+        torch.cuda.synchronize()
+        assert torch.equal(m.k[layer], kc) and torch.equal(m.v[layer], vc)
+        assert torch.equal(out.view(B, Hq, D), want)
+
+    for batch in (ids, ["c", "a"], ["a", "b"]):
+        one = m.begin_forward(batch, [1] * len(batch))
+        two = m.begin_forward(batch[:1], [1])  # another forward's plan in between
+        step(one, batch, 0)
+        step(two, batch[:1], 0)
+        step(one, batch, -1)
+        m.end_forward(one)

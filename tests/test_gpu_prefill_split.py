@@ -12,8 +12,8 @@ from test_gpu_kernels import ATOL, RTOL, _prefill_case
 DEV = "cuda:0"
 
 CASES = [  # lens, new tokens, Hq, Hkv, D, page size
-    ([512], [1], 32, 8, 128, 16),               # the shortest sequence that is cut
-    ([513], [17], 32, 8, 128, 16),              # a last run of one key
+    ([768], [1], 32, 8, 128, 16),               # the shortest sequence that is cut
+    ([769], [17], 32, 8, 128, 16),              # a last run of one key
     ([4096 + 31], [31], 8, 8, 128, 1),          # G = 1, 32 runs across two page-id windows
     ([6000, 300, 900], [33, 0, 5], 32, 8, 128, 16),
     ([1600, 1500], [150, 70], 16, 1, 128, 48),  # G = 16
