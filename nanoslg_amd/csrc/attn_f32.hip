@@ -26,8 +26,8 @@
 // prefill_f32_kernel: 64 rows (4 waves x 16) of one (sequence, KV head), K/V tiles staged
 //   in LDS once for all four. Bound by the matrix instructions (a tile of 32 keys is 4096
 //   cycles of a SIMD; two waves on it take ~10000 for both): 8 x 512 tokens over 512 keys
-//   1808 -> 543-575 us (92 of the 153 TFLOP/s that a large fp32 product reaches), one of
-//   512 from zero 145 -> 57, 64 over 4000 631 -> 63.
+//   1808 -> 500 us (103 of the 153 TFLOP/s that a large fp32 product reaches), one of 512
+//   from zero 145 -> 59, 64 over 4000 631 -> 63; 8 tokens, all latency, 8.9 and 9.3.
 // Both cut their keys into runs where there are too few workgroups; the runs' rows are
 // combined by merge_f32_kernel.
 //
@@ -304,36 +304,6 @@ __global__ void __launch_bounds__(64 * kWavesD) decode_f32_kernel(AttnF32Args p)
 
 // ---- prefill --------------------------------------------------------------------------
 
-// Wave-wide search for the (sequence, row tile) of tile slot g.
-__device__ inline bool locate_f32(const AttnF32Args& p, int g, int& b, int& tile) {
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  for (int s0 = 0; s0 < p.batch; s0 += 64) {
-    const int s = s0 + lane;
-    int nt = 0;
-    if (s < p.batch) {
-      const int n = p.qo_indptr[s + 1] - p.qo_indptr[s];
-      nt = n > 0 ? (n * p.group + kRowsP - 1) / kRowsP : 0;
-    }
-    int incl = nt;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int y = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += y;
-    }
-    const int excl = incl - nt;
-    const unsigned long long m = __ballot(nt > 0 && g >= base + excl && g < base + incl);
-    if (m) {
-      const int src = __ffsll((long long)m) - 1;
-      b = s0 + src;
-      tile = g - base - __shfl(excl, src, 64);
-      return true;
-    }
-    base += __shfl(incl, 63, 64);
-  }
-  return false;
-}
-
 template <int D, int kGroups>
 __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args p) {
   constexpr int NT = D / 16;
@@ -354,23 +324,18 @@ __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args 
   const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);   // rows 16 wave .. + 15 of the tile
   const int group_keys = kWaveKeys * __builtin_amdgcn_readfirstlane(tid >> 8);  // the wave's keys of an LDS tile
   const int r = lane & 15, gq = lane >> 4;
-  // Slots of one tile position follow each other over (KV head, run), the last tiles
-  // (most keys) first; empty slots of the grid's upper bound before them.
+  // work item: the tile's slot (longest first, empty ones last), then (run, KV head) in turn
   if (p.q_rows)
     zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, p.batch, p.out, p.out_stride * 4, p.num_qo_heads * D * 4,
                   blockIdx.x * (kThreads / 64) + (tid >> 6), gridDim.x * (kThreads / 64));
   const int runs = p.num_kv_heads * p.splits;
   const int run = blockIdx.x % runs;
   const int split = run / p.num_kv_heads, h = run - split * p.num_kv_heads;  // a head's runs on one XCD
-  int b = 0, tile = 0;
-  if (!locate_f32(p, p.row_tiles - 1 - (int)(blockIdx.x / runs), b, tile)) return;  // uniform over the workgroup
-  b = __builtin_amdgcn_readfirstlane(b);
-  tile = __builtin_amdgcn_readfirstlane(tile);
-
+  PrefillSeq sq;
+  if (!locate_row_tile(p.qo_indptr, p.indptr, p.last_len, p.page_size, p.batch, p.group, kRowsP, blockIdx.x / runs, sq))
+    return;  // uniform over the workgroup
+  const int b = sq.b, tile = sq.tile, q0 = sq.q0, n_new = sq.n_new, L = sq.len;
   const int G = p.group, ps = p.page_size;
-  const int q0 = p.qo_indptr[b];
-  const int n_new = p.qo_indptr[b + 1] - q0;
-  const int L = kv_len_f32(p, b);
   const int start = L - n_new > 0 ? L - n_new : 0;
   const int nrows = n_new * G;
   const int last_row = min(tile * kRowsP + kRowsP, nrows) - 1;
@@ -445,7 +410,7 @@ __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args 
   if (kv_begin < kv_end) {
     fetch_pages(kv_begin);
     fetch_rows(kv_begin);
-    fetch_pages(kv_begin + kKeys);
+    if (kv_begin + kKeys < kv_end) fetch_pages(kv_begin + kKeys);
   }
   // Q is waited for here: pending at the loop's entry, its wait would sit in the loop and
   // hold for the next tile's rows too, every tile.
@@ -467,8 +432,13 @@ __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args 
     const int wkey0 = key0 + group_keys;
     if (wkey0 >= wave_end) continue;  // uniform over the wave
     f32x4 s[kWaveKeys / 16];
+    // the wave's last tile may need one of its two 16-key halves only (16 tokens 11.0 ->
+    // 9.7 us, prompts of 300 to 600 111 -> 92 with the longest tiles first)
+    auto seen = [&](int k) { return k == 0 || wkey0 + 16 * k < wave_end; };  // uniform over the wave
 #pragma unroll
     for (int k = 0; k < kWaveKeys / 16; ++k) {
+      s[k] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (!seen(k)) break;
       f32x4 kt[NT];
 #pragma unroll
       for (int i = 0; i < NT; ++i)
@@ -486,7 +456,8 @@ __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args 
     }
     st.template softmax<kWaveKeys / 16>(s);
 #pragma unroll
-    for (int k = 0; k < kWaveKeys / 16; ++k)
+    for (int k = 0; k < kWaveKeys / 16; ++k) {
+      if (!seen(k)) break;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -496,6 +467,7 @@ __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args 
 #pragma unroll
           for (int e = 0; e < 4; ++e) st.o[4 * c + e] = mfma_f32(v[e], s[k][j], st.o[4 * c + e]);
         }
+    }
   }
 
   float l = rows_sum(st.l);
@@ -685,12 +657,10 @@ int attention_f32(const AttnF32Args& a, int32_t head_dim, hipStream_t s) {
   }
   dim3 grid;
   if (a.qo_indptr) {
-    // row-tile slots per (KV head, run): an upper bound over the batch (every sequence
-    // may end in a partial tile)
+    // row-tile slots: an upper bound over the batch (every sequence may end in a partial tile)
     const int64_t tiles = (a.total_q * a.group + kRowsP - 1) / kRowsP + a.batch;
     const int64_t wgs = tiles * a.num_kv_heads * a.splits;
     if (wgs > 0x7fffffff / 8) return fail(NSLG_EUNSUPPORTED, "attention_f32: too many rows");
-    p.row_tiles = (int32_t)tiles;
     grid = dim3((unsigned)wgs);
   } else {
     const int64_t wgs = (int64_t)a.batch * a.num_kv_heads;

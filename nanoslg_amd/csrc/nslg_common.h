@@ -242,10 +242,14 @@ __device__ inline bool locate_row_tile(const int32_t* qo, const int32_t* indptr,
       tile = nt - 1 - r;
     } else {
       int incl = nt;
+      if (batch <= 32) {  // a few lane reads are over sooner than the six rounds through LDS
+        for (int i = 0; i < batch - 1; ++i) incl += lane > i ? __builtin_amdgcn_readlane(nt, i) : 0;
+      } else {
 #pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const int y = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += y;
+        for (int off = 1; off < 64; off <<= 1) {
+          const int y = __shfl_up(incl, off, 64);
+          if (lane >= off) incl += y;
+        }
       }
       src = __ffsll((long long)__ballot(k >= incl - nt && k < incl)) - 1;
       tile = incl - 1 - k;
@@ -317,7 +321,7 @@ struct AttnF32Args {
   int64_t v_new_stride = 0;
   int32_t splits;              // runs of keys per row tile (1: no partials)
   void* workspace = nullptr;   // splits > 1: attention_f32_workspace bytes
-  int32_t row_tiles = 0;       // these are set by attention_f32
+  // set by attention_f32
   float* part_o = nullptr;     // [splits, total_q, Hq, D] partial outputs
   float* part_ml = nullptr;    // [splits, total_q, Hq, 2] running max and sum
 };
