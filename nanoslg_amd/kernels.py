@@ -1068,7 +1068,8 @@ def paged_prefill(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int, max_q:
     With q_rows (int32 [total_q] on the device) q and the result are the forward's
     padded grid of B * grid_width rows instead (nslg_paged_prefill_grid): ragged row t
     is grid row q_rows[t], sequence b's rows contiguous in its block of grid_width
-    rows, and the rows holding no token come out as zeros."""
+    rows, and the rows holding no token come out as zeros. `workspace` is not used: a
+    call that needs scratch (its keys cut into runs) allocates it on the current stream."""
     _require_gpu(q, qo_indptr, k_layer, v_layer, kv_indptr, kv_indices, kv_last_page_len)
     if q_rows is not None:
         _require_gpu(q, q_rows)

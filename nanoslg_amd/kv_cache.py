@@ -1837,7 +1837,7 @@ class ContiguousCacheContext(CacheContext):
         cache, plan = self.cache, self._plan
         B, S = q.shape[0], q.shape[1]
         if self._in_one_launch(S, q, k_new, v_new):
-            return self._decode(q)(layer_idx % cache.cfg.num_layers, q, k_new, v_new)
+            return self._decode(q)(self._layer(layer_idx), q, k_new, v_new)
         k_layer, v_layer = cache.paged_view(layer_idx)
         if not (self._is_decode and S == 1):
             # the write and the attention in one launch (a sequence's slot is its one page)
@@ -1863,12 +1863,15 @@ class ContiguousCacheContext(CacheContext):
             raise IndexError(f"position {self.max_kv_len - 1} is outside the rope tables ({cos.shape[0]} rows)")
         S = q.shape[1]
         if self._in_one_launch(S, q, k_new, v_new):
-            return self._decode(q)(layer_idx % cache.cfg.num_layers, q, k_new, v_new,
-                                   rope=(cos, sin, plan.pos_for(S)))
+            return self._decode(q)(self._layer(layer_idx), q, k_new, v_new, rope=(cos, sin, plan.pos_for(S)))
         k_layer, v_layer = cache.paged_view(layer_idx)
         q_rot = cache.kernels.rope_append(q, k_new, v_new, plan.pos_for(S), plan.slots_for(S), cos, sin,
                                           k_layer, v_layer)
         return self._attend_written(q_rot, k_layer, v_layer)
+
+    def _layer(self, layer_idx):
+        """A layer index as the pool tensors take it (negative ones from the end)."""
+        return layer_idx if layer_idx >= 0 else layer_idx + self.cache.cfg.num_layers
 
     def _in_one_launch(self, S, q, k_new, v_new):
         """A decode step whose rows the decode launch writes itself (a padded step's row,

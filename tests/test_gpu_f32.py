@@ -101,4 +101,8 @@ def test_contiguous_decode_in_one_launch(dtype):
         step(one, batch, 0)
         step(two, batch[:1], 0)
         step(one, batch, -1)
+        q, kv = rnd(len(batch), 1, Hq, D), rnd(len(batch), 1, Hkv, D)
+        for bad in (L, -L - 1):
+            with pytest.raises(IndexError):
+                one.attend(bad, q, kv, kv, Hq, Hkv)
         m.end_forward(one)
