@@ -100,3 +100,23 @@ def test_pad_rows_shared_by_the_launch(news, W, dtype, D):
         want[at] = K.paged_prefill(q[at].contiguous(), d(qo), T, max(news), *plan)
     torch.cuda.synchronize()
     assert torch.equal(out, want)
+
+
+ORDERS = [  # new tokens per sequence (each over a few cached keys)
+    [300, 256, 310, 290],                       # near-uniform tile counts: rounds, one sequence short of a tile
+    [700, 1, 0, 64, 65, 300],                   # sequence by sequence; none, one and several tiles
+    [(7 * i) % 90 for i in range(40)],          # more than 32 sequences
+    [(11 * i) % 70 + 1 for i in range(70)],     # more than 64 sequences
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("case", range(len(ORDERS)))
+def test_every_row_tile_is_taken_once(case, dtype):
+    """Every order of the row tiles against the oracle: a tile left out leaves its rows
+    unwritten."""
+    from test_gpu_kernels import F32_TOL
+    news = ORDERS[case]
+    out, ref = _prefill_case([n + 5 for n in news], news, 8, 2, 64, 16, dtype, seed=760 + case)
+    torch.testing.assert_close(out, ref, **(F32_TOL if dtype == torch.float32 else dict(atol=ATOL, rtol=RTOL)))
