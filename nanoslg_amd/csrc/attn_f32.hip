@@ -511,7 +511,9 @@ __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args 
 
 // Log-sum-exp merge of the runs of each (query token, query head) row: D / 4 lanes per
 // row, one float4 each, and kParts such groups of lanes, 16 runs each (one after the
-// other, 63 runs took 9.7 us). A run without a key of the row has sum 0.
+// other, 63 runs took 9.7 us). A run without a key of the row has sum 0 and is passed
+// over (its rows may be unwritten); one whose scores are all NaN has max -inf and sum NaN,
+// and its weight is NaN.
 template <int D, int kParts>
 __global__ void __launch_bounds__(kParts * (D / 4) < 256 ? 256 : kParts * (D / 4)) merge_f32_kernel(AttnF32Args p) {
   constexpr int kLanes = D / 4;
@@ -537,10 +539,11 @@ __global__ void __launch_bounds__(kParts * (D / 4) < 256 ? 256 : kParts * (D / 4
   for (int i = 0; i < kParts; ++i) m = fmaxf(m, ml[i].x);
 #pragma unroll
   for (int off = 1; off < 16; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 16));
-  float f = 0.f, l = 0.f;  // the weight of the part's run sl; the row's sum
+  float f = -1.f, l = 0.f;  // the weight of the part's run sl (-1: no key); the row's sum
 #pragma unroll
   for (int i = 0; i < kParts; ++i) {
-    const float w = ml[i].y == 0.f ? 0.f : expf(ml[i].x - m);
+    if (ml[i].y == 0.f) continue;
+    const float w = ml[i].y != ml[i].y ? ml[i].y : expf(ml[i].x - m);
     if (i == part) f = w;
     l = fmaf(w, ml[i].y, l);
   }
@@ -556,8 +559,8 @@ __global__ void __launch_bounds__(kParts * (D / 4) < 256 ? 256 : kParts * (D / 4
       o[u] = *reinterpret_cast<const f32x4*>(p.part_o + (min(s0 + u, s_end - 1) * rows + prow) * D + d);
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const float fs = s0 + u < s_end ? __shfl(f, (s0 + u) & 15, 16) : 0.f;
-      if (fs == 0.f) continue;  // (a run without keys left no rows)
+      const float fs = s0 + u < s_end ? __shfl(f, (s0 + u) & 15, 16) : -1.f;
+      if (fs < 0.f) continue;  // a run without keys left no rows
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[e] = fmaf(fs, o[u][e], acc[e]);
     }

@@ -1,11 +1,13 @@
 """The fp32 attention kernels at the edges of their tiles, waves, runs and pages, against
 the oracle's fp32 SDPA (within summation-order differences), and the decode's fused write
 of the new rows against append_kv."""
+import math
+
 import numpy as np
 import pytest
 import torch
 
-from test_gpu_kernels import F32_TOL, _csr_random, _decode_case, _prefill_case
+from test_gpu_kernels import ATOL, F32_TOL, RTOL, _csr_random, _decode_case, _prefill_case
 
 DEV = "cuda:0"
 
@@ -106,3 +108,50 @@ def test_contiguous_decode_in_one_launch(dtype):
             with pytest.raises(IndexError):
                 one.attend(bad, q, kv, kv, Hq, Hkv)
         m.end_forward(one)
+
+
+def _attention64(q, k, v, n):
+    """Causal attention of the last n tokens, bottom-right aligned, in 64 bits: q [n, Hq, D]
+    over k, v [m, Hkv, D]; a NaN or infinity goes where softmax and product take it."""
+    q, k, v = (x.double().transpose(0, 1) for x in (q, k, v))
+    G, m = q.shape[0] // k.shape[0], k.shape[1]
+    s = q @ k.repeat_interleave(G, 0).transpose(1, 2) / math.sqrt(q.shape[2])
+    seen = torch.arange(m)[None] <= torch.arange(m - n, m)[:, None]
+    p = torch.softmax(s.masked_fill(~seen, -math.inf), -1)
+    return (p @ v.repeat_interleave(G, 0)).transpose(0, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L,n", [(900, 0), (4000, 0), (900, 3), (1300, 40)])  # n = 0: a decode token
+@pytest.mark.parametrize("bad", ["nan", "nan_row", "inf"])
+def test_nonfinite_keys_reach_the_rows_that_see_them(bad, L, n, dtype):
+    """Whole runs of keys, or one key, that score NaN or +-inf, in calls cut into runs and
+    merged: a row of the KV head is NaN where softmax over its keys is, and no other is."""
+    from nanoslg_amd import kernels as K
+    Hq, Hkv, D, ps = 8, 2, 128, 16
+    g = torch.Generator().manual_seed(L + n)
+    q = torch.randn(max(n, 1), Hq, D, generator=g).to(dtype)
+    k, v = (torch.randn(L, Hkv, D, generator=g).to(dtype) for _ in range(2))
+    if bad == "nan":
+        k[:512, 1] = math.nan     # all the keys of the first runs (64 or 128 keys, or key tiles of 128)
+    elif bad == "nan_row":
+        k[700, 1, 5] = math.nan
+    else:
+        k[3, 1, 5] = math.inf     # +inf or -inf by the sign of the row's element 5
+    npg = -(-L // ps)
+    pool = torch.zeros(2, npg * ps, Hkv, D, dtype=dtype)
+    pool[0, :L], pool[1, :L] = k, v
+    kp, vp = pool.view(2, npg, ps, Hkv, D).to(DEV)
+    i32 = lambda *a: torch.tensor(a, dtype=torch.int32, device=DEV)  # noqa: E731
+    plan = (i32(0, npg), torch.arange(npg, dtype=torch.int32, device=DEV), i32((L - 1) % ps + 1))
+    if n:
+        out = K.paged_prefill(q.to(DEV), i32(0, n), n, n, kp, vp, *plan)
+    else:
+        out = K.paged_decode(q.to(DEV), kp, vp, *plan, npg)
+    ref = _attention64(q, k, v, max(n, 1))
+    out = out.cpu()
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert ref[:, :Hq // Hkv].isfinite().all() and ref.isnan().any()
+    tol = F32_TOL if dtype == torch.float32 else dict(atol=ATOL, rtol=RTOL)
+    torch.testing.assert_close(out.float(), ref.float(), equal_nan=True, **tol)
