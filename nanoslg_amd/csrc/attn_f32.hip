@@ -573,7 +573,10 @@ __global__ void __launch_bounds__(kParts * (D / 4) < 256 ? 256 : kParts * (D / 4
 #pragma unroll
     for (int i = 0; i < kParts - 1; ++i) acc += mine[i * kLanes];
   }
-  if (row0 >= rows || (p.qo_indptr && t >= p.qo_indptr[p.batch])) return;  // (a row of no sequence has no runs)
+  if (row0 >= rows) return;
+  // (a row of no sequence has no runs: past the last's, or before the first's in a batch
+  // that is part of a larger one)
+  if (p.qo_indptr && (t < p.qo_indptr[0] || t >= p.qo_indptr[p.batch])) return;
   const int64_t orow = f32_grid_row(p, t);
   if (orow < 0) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;

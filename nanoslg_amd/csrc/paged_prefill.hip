@@ -705,7 +705,9 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(PrefillParams p) {
   const int64_t pr = (int64_t)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
   if (pr >= rows) return;
   const int t = (int)(pr / p.num_qo_heads);
-  if (t >= p.qo_indptr[p.batch]) return;  // a row of no sequence: nothing was left for it
+  // a row of no sequence (past the last's, or before the first's in a batch that is part of
+  // a larger one): nothing was left for it
+  if (t < p.qo_indptr[0] || t >= p.qo_indptr[p.batch]) return;
   // Every lane of a 16-lane group loads two runs' (max, sum) together with the count, so
   // the row takes two rounds of loads whatever its runs (run by run, 17 runs took 20 us).
   const int s_lane = threadIdx.x & 15;

@@ -120,3 +120,33 @@ def test_every_row_tile_is_taken_once(case, dtype):
     news = ORDERS[case]
     out, ref = _prefill_case([n + 5 for n in news], news, 8, 2, 64, 16, dtype, seed=760 + case)
     torch.testing.assert_close(out, ref, **(F32_TOL if dtype == torch.float32 else dict(atol=ATOL, rtol=RTOL)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_rows_of_no_sequence_are_left_alone(dtype):
+    """A call on part of a larger batch's ragged rows (qo_indptr starts past row 0), cut into
+    runs: the part's rows as in a call of their own, the rows before and after unwritten,
+    whatever the scratch held."""
+    from nanoslg_amd import kernels as K
+    Hq, Hkv, D, ps, lens, news, first = 8, 2, 128, 16, [1500, 900], [20, 7], 11
+    g = torch.Generator().manual_seed(3)
+    npg = [-(-n // ps) for n in lens]
+    k, v = (torch.randn(sum(npg), ps, Hkv, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+    q = torch.randn(first + sum(news) + 5, Hq, D, generator=g).to(dtype).to(DEV)
+    d = lambda *a: torch.tensor(a, dtype=torch.int32, device=DEV)  # noqa: E731
+    plan = (k, v, d(0, npg[0], sum(npg)), torch.arange(sum(npg), dtype=torch.int32, device=DEV),
+            d(*[(n - 1) % ps + 1 for n in lens]))
+    T = sum(news)
+    last = first + T
+    # the same scratch bytes again, every count and sum in it 2 or more
+    need = K._prefill_workspace(q, 2, Hq, D, last, max(news), max(lens))[2]
+    assert need > 256
+    torch.cuda.synchronize()
+    torch.full((need,), 0x40, dtype=torch.uint8, device=DEV)
+    out = torch.full_like(q, 7.0)
+    K.paged_prefill(q, d(first, first + news[0], last), last, max(news), *plan, out=out)
+    want = K.paged_prefill(q[first:last].contiguous(), d(0, news[0], T), T, max(news), *plan)
+    torch.cuda.synchronize()
+    assert (out[:first] == 7).all() and (out[last:] == 7).all()
+    torch.testing.assert_close(out[first:last], want, atol=ATOL, rtol=RTOL)
