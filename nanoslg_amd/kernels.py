@@ -764,6 +764,14 @@ class DecodeLaunch:
         self._ws_pages = bound
         return self
 
+    def bound_to(self, slot_mapping: torch.Tensor, kv_indptr: torch.Tensor, kv_indices: torch.Tensor,
+                 kv_last_page_len: torch.Tensor, total_pages: int) -> "DecodeLaunch":
+        """A second launcher of the same pools, batch size and head count for another
+        forward's plan (not checked again), this one staying bound to its own."""
+        other = object.__new__(type(self))
+        other.__dict__.update(self.__dict__)
+        return other.rebind(slot_mapping, kv_indptr, kv_indices, kv_last_page_len, total_pages, check=False)
+
     def _kv_rows(self, t: torch.Tensor, name: str) -> int:
         """Row stride of k_new / v_new: [B, ..., Hkv, D] rows of one token each."""
         sh = t.shape

@@ -1881,23 +1881,19 @@ class ContiguousCacheContext(CacheContext):
 
     def _decode(self, q):
         """The forward's decode launcher (kernels.DecodeLaunch) over the slots, each a page
-        of max_seq_len tokens; the previous forward's, re-bound, when batch and heads stay."""
+        of max_seq_len tokens. A launcher belongs to one forward and is bound once, so
+        forwards of one cache can be attended in any order, from several threads too."""
         cache, plan = self.cache, self._plan
         launch = self._decode_launch
         if launch is None:
-            launch, kern = cache._launcher, cache.kernels
-            if (launch is not None and hasattr(launch, "rebind") and launch.B == plan.batch
-                    and launch.Hq == q.shape[2] and launch.pools[0] is cache.k and launch.pools[1] is cache.v):
-                launch.rebind(plan.slot, plan.indptr, plan.indices, plan.lpl, plan.total_pages, check=False)
+            prev, kern = cache._launcher, cache.kernels
+            args = (plan.slot, plan.indptr, plan.indices, plan.lpl, plan.total_pages)
+            if (prev is not None and hasattr(prev, "bound_to") and prev.B == plan.batch
+                    and prev.Hq == q.shape[2] and prev.pools[0] is cache.k and prev.pools[1] is cache.v):
+                launch = prev.bound_to(*args)
             else:
-                launch = cache._launcher = kern.DecodeLaunch(cache.k, cache.v, plan.slot, plan.indptr, plan.indices,
-                                                             plan.lpl, plan.total_pages, q.shape[2],
-                                                             workspace=cache.workspace)
-            launch.bound_plan = plan
-            self._decode_launch = launch
-        elif launch.bound_plan is not plan:  # another forward was begun since
-            launch.rebind(plan.slot, plan.indptr, plan.indices, plan.lpl, plan.total_pages, check=False)
-            launch.bound_plan = plan
+                launch = kern.DecodeLaunch(cache.k, cache.v, *args, q.shape[2], workspace=cache.workspace)
+            self._decode_launch = cache._launcher = launch
         return launch
 
     def _attend_written(self, q, k_layer, v_layer):
@@ -1934,7 +1930,7 @@ class ContiguousKVCache(KVCacheManager):
         self.states: Dict[str, _ContigSeqState] = {}
         self._slot = 0
         self.workspace = self.kernels.Workspace(self.device, 16 << 20)
-        self._launcher = None  # the last decode forward's kernels.DecodeLaunch
+        self._launcher = None  # the last decode forward's kernels.DecodeLaunch: the next one's is made from it
 
     def paged_view(self, layer_idx):
         return self.k[layer_idx], self.v[layer_idx]

@@ -155,3 +155,43 @@ def test_nonfinite_keys_reach_the_rows_that_see_them(bad, L, n, dtype):
     assert ref[:, :Hq // Hkv].isfinite().all() and ref.isnan().any()
     tol = F32_TOL if dtype == torch.float32 else dict(atol=ATOL, rtol=RTOL)
     torch.testing.assert_close(out.float(), ref.float(), equal_nan=True, **tol)
+
+
+@pytest.mark.gpu
+def test_contiguous_forwards_attended_in_between(monkeypatch):
+    """A decode forward of the contiguous cache attended while another one's call is under
+    way (between its launcher being found and its launch, as from a second thread): each
+    writes and reads the slots of its own sequences."""
+    from nanoslg_amd import kernels as K
+    from nanoslg_amd.kv_cache import ContiguousKVCache, KVCacheConfig
+    Hq, Hkv, D = 8, 2, 64
+    m = ContiguousKVCache(KVCacheConfig(num_layers=1, num_kv_heads=Hkv, num_qo_heads=Hq, head_dim=D, max_batch_size=3,
+                                        max_seq_len=80, dtype=torch.float32, device=torch.device(DEV),
+                                        backend="contiguous"))
+    g = torch.Generator().manual_seed(6)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(DEV)  # noqa: E731
+    for s in "abc":
+        m.allocate_sequence(s)
+    ctx = m.begin_forward(list("abc"), [40, 3, 70])
+    ctx.attend(0, rnd(3, 70, Hq, D), rnd(3, 70, Hkv, D), rnd(3, 70, Hkv, D), Hq, Hkv)
+    m.end_forward(ctx)
+    forwards = [m.begin_forward([s], [1]) for s in "abc"]
+    inputs = [(rnd(1, 1, Hq, D), rnd(1, 1, Hkv, D), rnd(1, 1, Hkv, D)) for _ in forwards]
+    kc, vc = m.k[0].clone(), m.v[0].clone()
+    want = []
+    for f, (q, k, v) in zip(forwards, inputs):
+        K.append_kv(k, v, f._plan.slot, kc, vc)
+        want.append(K.paged_decode(q[:, 0], kc, vc, f._plan.indptr, f._plan.indices, f._plan.lpl, 1).view(1, 1, -1))
+    forwards[2].attend(0, *inputs[2], Hq, Hkv)  # (an earlier forward of the same batch size)
+    got, call = [], K.DecodeLaunch.__call__
+
+    def nested(self, *args, **kw):
+        monkeypatch.setattr(K.DecodeLaunch, "__call__", call)
+        got.append(forwards[1].attend(0, *inputs[1], Hq, Hkv))
+        return call(self, *args, **kw)
+
+    monkeypatch.setattr(K.DecodeLaunch, "__call__", nested)
+    got.insert(0, forwards[0].attend(0, *inputs[0], Hq, Hkv))
+    torch.cuda.synchronize()
+    assert torch.equal(m.k[0], kc) and torch.equal(m.v[0], vc)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
