@@ -1835,10 +1835,10 @@ class ContiguousCacheContext(CacheContext):
 
     def attend(self, layer_idx, q, k_new, v_new, n_heads, n_kv_heads):
         cache, plan = self.cache, self._plan
-        B, S = q.shape[0], q.shape[1]
-        if self._in_one_launch(S, q, k_new, v_new):
+        if self._in_one_launch(layer_idx, q, k_new, v_new):
             return self._decode(q)(self._layer(layer_idx), q, k_new, v_new)
         k_layer, v_layer = cache.paged_view(layer_idx)
+        B, S = q.shape[0], q.shape[1]
         if not (self._is_decode and S == 1):
             # the write and the attention in one launch (a sequence's slot is its one page)
             uniform = self._uniform_rows and S == self._iw
@@ -1861,10 +1861,11 @@ class ContiguousCacheContext(CacheContext):
         cache, plan = self.cache, self._plan
         if self.max_kv_len > cos.shape[0]:
             raise IndexError(f"position {self.max_kv_len - 1} is outside the rope tables ({cos.shape[0]} rows)")
-        S = q.shape[1]
-        if self._in_one_launch(S, q, k_new, v_new):
-            return self._decode(q)(self._layer(layer_idx), q, k_new, v_new, rope=(cos, sin, plan.pos_for(S)))
+        if (self._in_one_launch(layer_idx, q, k_new, v_new)
+                and cos.get_device() == sin.get_device() == q.get_device()):
+            return self._decode(q)(self._layer(layer_idx), q, k_new, v_new, rope=(cos, sin, plan.pos_for(1)))
         k_layer, v_layer = cache.paged_view(layer_idx)
+        S = q.shape[1]
         q_rot = cache.kernels.rope_append(q, k_new, v_new, plan.pos_for(S), plan.slots_for(S), cos, sin,
                                           k_layer, v_layer)
         return self._attend_written(q_rot, k_layer, v_layer)
@@ -1873,28 +1874,50 @@ class ContiguousCacheContext(CacheContext):
         """A layer index as the pool tensors take it (negative ones from the end)."""
         return layer_idx if layer_idx >= 0 else layer_idx + self.cache.cfg.num_layers
 
-    def _in_one_launch(self, S, q, k_new, v_new):
-        """A decode step whose rows the decode launch writes itself (a padded step's row,
-        and tensors of another type, take the separate calls)."""
-        return (self._is_decode and S == 1 and self._iw == 1
-                and q.dtype == k_new.dtype == v_new.dtype == self.cache.cfg.dtype)
+    def _in_one_launch(self, layer_idx, q, k_new, v_new):
+        """A decode step whose rows the decode launch writes itself: one row a sequence, of
+        the pool's dtype and device, q [B, 1, Hq, D] and k_new / v_new [B, 1, Hkv, D] at row
+        strides that do not overlap, q 16-byte aligned. A padded step's row and all other
+        forms take the separate calls, which serve or refuse each as they always did."""
+        if not (self._is_decode and self._iw == 1 and type(layer_idx) is int):
+            return False
+        pool, B = self.cache.k, self.batch_size
+        Hkv, D = pool.shape[3], pool.shape[4]
+        dt, dev = pool.dtype, pool.get_device()
+        if not (q.dtype == k_new.dtype == v_new.dtype == dt
+                and q.get_device() == k_new.get_device() == v_new.get_device() == dev):
+            return False
+        qs, row = q.shape, (B, 1, Hkv, D)
+        if (len(qs) != 4 or qs[0] != B or qs[1] != 1 or qs[3] != D or qs[2] % Hkv or k_new.shape != row
+                or v_new.shape != row):
+            return False
+        st, sk, sv = q.stride(), k_new.stride(), v_new.stride()
+        return (st[3] == sk[3] == sv[3] == 1 and st[2] == sk[2] == sv[2] == D and st[0] >= qs[2] * D
+                and sk[0] >= Hkv * D and sv[0] >= Hkv * D
+                and not (q.data_ptr() | st[0] * q.element_size()) & 15)
 
     def _decode(self, q):
         """The forward's decode launcher (kernels.DecodeLaunch) over the slots, each a page
         of max_seq_len tokens. A launcher belongs to one forward and is bound once, so
-        forwards of one cache can be attended in any order, from several threads too."""
+        forwards of one cache can be attended in any order, from several threads too;
+        calls with other heads or after the pools moved get a new one."""
         cache, plan = self.cache, self._plan
         launch = self._decode_launch
-        if launch is None:
+        if launch is None or not self._serves(launch, q):
             prev, kern = cache._launcher, cache.kernels
             args = (plan.slot, plan.indptr, plan.indices, plan.lpl, plan.total_pages)
-            if (prev is not None and hasattr(prev, "bound_to") and prev.B == plan.batch
-                    and prev.Hq == q.shape[2] and prev.pools[0] is cache.k and prev.pools[1] is cache.v):
+            if prev is not None and hasattr(prev, "bound_to") and prev.B == plan.batch and self._serves(prev, q):
                 launch = prev.bound_to(*args)
             else:
                 launch = kern.DecodeLaunch(cache.k, cache.v, *args, q.shape[2], workspace=cache.workspace)
             self._decode_launch = cache._launcher = launch
         return launch
+
+    def _serves(self, launch, q):
+        """Whether a launcher made for these pools and heads is one for q's and the cache's."""
+        cache = self.cache
+        return not hasattr(launch, "bound_to") or (
+            launch.Hq == q.shape[2] and launch.kp0 == cache.k.data_ptr() and launch.vp0 == cache.v.data_ptr())
 
     def _attend_written(self, q, k_layer, v_layer):
         """Attention of the forward's rows over the slots (K/V already written)."""

@@ -195,3 +195,71 @@ def test_contiguous_forwards_attended_in_between(monkeypatch):
     torch.cuda.synchronize()
     assert torch.equal(m.k[0], kc) and torch.equal(m.v[0], vc)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+FORMS = ["heads", "shared_kv", "flat_kv", "heads_apart", "one_head", "cpu_sin", "cpu_q", "f64_k"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("form", FORMS)
+def test_contiguous_decode_takes_the_forms_of_the_separate_calls(form, rope):
+    """A decode step of the contiguous cache serves what append_kv (rope_append) and
+    paged_decode serve, with their result, and refuses with their error what they refuse:
+    other query heads in one forward, one K row for the whole batch, rows of other ranks,
+    heads apart in memory, tensors of another device or dtype."""
+    from nanoslg_amd import kernels as K
+    from nanoslg_amd.kv_cache import ContiguousKVCache, KVCacheConfig
+    Hq, Hkv, D, B = (1, 1, 64, 2) if form == "one_head" else (8, 2, 64, 2)
+    m = ContiguousKVCache(KVCacheConfig(num_layers=1, num_kv_heads=Hkv, num_qo_heads=Hq, head_dim=D, max_batch_size=B,
+                                        max_seq_len=80, dtype=torch.float16, device=torch.device(DEV),
+                                        backend="contiguous"))
+    g = torch.Generator().manual_seed(6)
+    rnd = lambda *s: torch.randn(*s, generator=g).half().to(DEV)  # noqa: E731
+    for s in "ab":
+        m.allocate_sequence(s)
+    ctx = m.begin_forward(["a", "b"], [40, 3])
+    ctx.attend(0, rnd(B, 40, Hq, D), rnd(B, 40, Hkv, D), rnd(B, 40, Hkv, D), Hq, Hkv)
+    m.end_forward(ctx)
+    ctx = m.begin_forward(["a", "b"], [1, 1])
+    cos, sin = (torch.randn(80, D, generator=g).to(DEV) for _ in range(2))
+    q, k, v = rnd(B, 1, Hq, D), rnd(B, 1, Hkv, D), rnd(B, 1, Hkv, D)
+    if form == "heads":
+        (ctx.attend_rope(0, q, k, v, cos, sin, Hq, Hkv) if rope else ctx.attend(0, q, k, v, Hq, Hkv))
+        q = rnd(B, 1, 2 * Hq, D)
+    elif form == "shared_kv":
+        k, v = k[:1].expand(B, 1, Hkv, D), v[:1].expand(B, 1, Hkv, D)
+    elif form == "flat_kv":
+        k, v = k[:, 0], v[:, 0]
+    elif form == "heads_apart":
+        q = rnd(B, Hq, 3, D).transpose(1, 2)[:, :1]
+    elif form == "one_head":
+        q = rnd(B, Hq, 3, D).transpose(1, 2)[:, :1]
+    elif form == "cpu_sin":
+        sin = sin.cpu()
+    elif form == "cpu_q":
+        q = q.cpu()
+    else:
+        k = k.double()
+
+    def separate(kc, vc):
+        p = ctx._plan
+        if rope:
+            r = K.rope_append(q, k, v, p.pos_for(1), p.slots_for(1), cos, sin, kc, vc)
+        else:
+            K.append_kv(k, v, p.slots_for(1), kc, vc)
+            r = q
+        return K.paged_decode(r[:, 0], kc, vc, p.indptr, p.indices, p.lpl, p.total_pages).view(B, 1, -1)
+
+    kc, vc = m.k[0].clone(), m.v[0].clone()
+    call = lambda: (ctx.attend_rope(0, q, k, v, cos, sin, Hq, Hkv) if rope  # noqa: E731
+                    else ctx.attend(0, q, k, v, Hq, Hkv))
+    try:
+        want = separate(kc, vc)
+    except (ValueError, TypeError, K._lib.KernelLibraryError) as e:
+        with pytest.raises(type(e)):
+            call()
+        return
+    out = call()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(m.k[0], kc) and torch.equal(m.v[0], vc)
