@@ -256,10 +256,19 @@ class Workspace:
         self.device = torch.device(device)
         self.buf = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=self.device)
 
+        self.prefill_buf: Optional[torch.Tensor] = None
+
     def get(self, nbytes: int) -> torch.Tensor:
         if self.buf.numel() < nbytes:
             self.buf = torch.zeros(int(nbytes * 1.25) + 256, dtype=torch.uint8, device=self.device)
         return self.buf
+
+    def get_prefill(self, nbytes: int) -> torch.Tensor:
+        """Scratch of prefill calls: memory of its own, since a chunk layout that a decode
+        call recorded in get()'s is read again after the calls in between."""
+        if self.prefill_buf is None or self.prefill_buf.numel() < nbytes:
+            self.prefill_buf = torch.empty(int(nbytes * 1.25) + 256, dtype=torch.uint8, device=self.device)
+        return self.prefill_buf
 
 
 class DecodeGroups:
@@ -906,11 +915,11 @@ _PREFILL_WS: Dict[Tuple[int, int, int, int, int], int] = {}  # nslg_paged_prefil
 PREFILL_SPLIT_KEYS = {64: 1024, 128: 768, 256: 768}
 
 
-def _prefill_workspace(q, B, Hq, D, total_q, max_q, max_kv):
+def _prefill_workspace(q, B, Hq, D, total_q, max_q, max_kv, workspace=None):
     """(owner, address, bytes) of the partials of a prefill call whose longest sequence has
-    max_kv keys; (None, None, 0) where the call takes its keys in one run. From the caching
-    allocator on the current stream, and not the cache's workspace: one cache's prefills
-    may run on another stream than its decodes."""
+    max_kv keys; (None, None, 0) where the call takes its keys in one run. In the caller's
+    workspace; without one, and for the caches, whose forwards may run on several streams
+    at once, from the caching allocator on the current stream."""
     if max_kv < PREFILL_SPLIT_KEYS.get(D, 1 << 62):
         return None, None, 0
     key = (B, Hq, D, total_q, max_q)
@@ -922,7 +931,7 @@ def _prefill_workspace(q, B, Hq, D, total_q, max_q, max_kv):
         _PREFILL_WS[key] = need
     if need <= 256:
         return None, None, 0
-    ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if workspace is None else workspace.get_prefill(need)
     return ws, ws.data_ptr(), need
 
 
@@ -1024,7 +1033,8 @@ def paged_prefill_append(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int,
     (nslg_paged_prefill_append; 16-bit pools). k_new / v_new: [..., Hkv, D] with q's
     rows (ragged [T] rows, or the B * grid_width grid rows with q_rows): token t of
     sequence b is written to position L_b - n_b + t through the block table. Returns
-    paged_prefill's result; the pool holds the rows, as after append_kv."""
+    paged_prefill's result; the pool holds the rows, as after append_kv. `workspace` as
+    for paged_prefill."""
     _require_gpu(q, qo_indptr, k_new, v_new, k_layer, v_layer, kv_indptr, kv_indices, kv_last_page_len)
     for t, name in ((qo_indptr, "qo_indptr"), (kv_indptr, "kv_indptr"), (kv_indices, "kv_indices"),
                     (kv_last_page_len, "kv_last_page_len")):
@@ -1053,7 +1063,7 @@ def paged_prefill_append(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int,
     lib = _lib.load()
     # the average sequence's table stands for the longest one (its length is on the device)
     max_kv = kv_indices.numel() * ps // max(B, 1)
-    ws, ws_ptr, ws_bytes = _prefill_workspace(q, B, Hq, D, int(total_q), int(max_q), max_kv)
+    ws, ws_ptr, ws_bytes = _prefill_workspace(q, B, Hq, D, int(total_q), int(max_q), max_kv, workspace)
     scale = (1.0 / math.sqrt(D)) if sm_scale is None else float(sm_scale)
     rc = lib.nslg_paged_prefill_append(q.data_ptr(), q.stride(0), qo_indptr.data_ptr(),
                                        None if q_rows is None else q_rows.data_ptr(), int(grid_width),
@@ -1076,8 +1086,9 @@ def paged_prefill(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int, max_q:
     With q_rows (int32 [total_q] on the device) q and the result are the forward's
     padded grid of B * grid_width rows instead (nslg_paged_prefill_grid): ragged row t
     is grid row q_rows[t], sequence b's rows contiguous in its block of grid_width
-    rows, and the rows holding no token come out as zeros. `workspace` is not used: a
-    call that needs scratch (its keys cut into runs) allocates it on the current stream."""
+    rows, and the rows holding no token come out as zeros. `workspace`: scratch for a call
+    whose keys are cut into runs (up to 34 MB), kept from call to call; one call at a time
+    may use it. Without it such a call allocates its scratch on the current stream."""
     _require_gpu(q, qo_indptr, k_layer, v_layer, kv_indptr, kv_indices, kv_last_page_len)
     if q_rows is not None:
         _require_gpu(q, q_rows)
@@ -1104,7 +1115,7 @@ def paged_prefill(q: torch.Tensor, qo_indptr: torch.Tensor, total_q: int, max_q:
     lib = _lib.load()
     # the average sequence's table stands for the longest one (its length is on the device)
     max_kv = kv_indices.numel() * ps // max(B, 1)
-    ws, ws_ptr, ws_bytes = _prefill_workspace(q, B, Hq, D, int(total_q), int(max_q), max_kv)
+    ws, ws_ptr, ws_bytes = _prefill_workspace(q, B, Hq, D, int(total_q), int(max_q), max_kv, workspace)
     scale = (1.0 / math.sqrt(D)) if sm_scale is None else float(sm_scale)
     if q_rows is not None:
         rc = lib.nslg_paged_prefill_grid(q.data_ptr(), q.stride(0), qo_indptr.data_ptr(), q_rows.data_ptr(),

@@ -150,3 +150,37 @@ def test_rows_of_no_sequence_are_left_alone(dtype):
     torch.cuda.synchronize()
     assert (out[:first] == 7).all() and (out[last:] == 7).all()
     torch.testing.assert_close(out[first:last], want, atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.gpu
+def test_a_callers_workspace_is_used():
+    """Calls cut into runs with the caller's workspace: nothing allocated but the output,
+    the result that of a call without one, and a chunk layout that a decode call recorded in
+    the workspace still read after them."""
+    from nanoslg_amd import kernels as K
+    Hq, Hkv, D, ps, L, n = 8, 2, 128, 16, 4000, 20
+    g = torch.Generator().manual_seed(4)
+    rnd = lambda *s: torch.randn(*s, generator=g).half().to(DEV)  # noqa: E731
+    k, v, q, dq = rnd(L // ps, ps, Hkv, D), rnd(L // ps, ps, Hkv, D), rnd(n, Hq, D), rnd(1, Hq, D)
+    kn, vn = k[-2:].reshape(-1, Hkv, D)[-n:].clone(), v[-2:].reshape(-1, Hkv, D)[-n:].clone()
+    d = lambda *a: torch.tensor(a, dtype=torch.int32, device=DEV)  # noqa: E731
+    plan = (d(0, L // ps), torch.arange(L // ps, dtype=torch.int32, device=DEV), d(ps))
+    qo, out = d(0, n), torch.empty_like(q)
+    ws = K.Workspace(DEV, 64 << 20)
+    want = K.paged_prefill(q, qo, n, n, k, v, *plan)
+    step = K.paged_decode(dq, k, v, *plan, L // ps, workspace=ws, layout=101)
+    before = ws.buf.clone()
+    for i in range(2):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        base = torch.cuda.memory_allocated()
+        K.paged_prefill(q, qo, n, n, k, v, *plan, out=out, workspace=ws)
+        peak = torch.cuda.max_memory_allocated() - base
+        assert i == 0 or peak == 0
+        assert torch.equal(out, want)
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    o2 = K.paged_prefill_append(q, qo, n, n, kn, vn, k, v, *plan, workspace=ws)
+    assert torch.cuda.max_memory_allocated() - base <= o2.numel() * 2 + 512
+    assert torch.equal(o2, want) and torch.equal(ws.buf, before)
+    assert torch.equal(K.paged_decode(dq, k, v, *plan, L // ps, workspace=ws, layout=-101), step)
