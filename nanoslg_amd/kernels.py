@@ -858,7 +858,7 @@ class DecodeLaunch:
             if pos.get_device() != di or pos.dtype != torch.int32 or pos.numel() != B or not pos.is_contiguous():
                 raise ValueError(f"DecodeLaunch: positions must be {B} contiguous int32 on {self.device}")
             cos, sin = _rope_tables(cos, sin, D)
-            if cos.get_device() != di:
+            if cos.get_device() != di or sin.get_device() != di:
                 raise ValueError(f"DecodeLaunch: rope tables must be on {self.device}")
             kn, vn = k_new.data_ptr(), v_new.data_ptr()
             cp, sp, cst = cos.data_ptr(), sin.data_ptr(), cos.stride(0)

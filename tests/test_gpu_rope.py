@@ -197,3 +197,18 @@ def test_decode_rope_append_equals_rope_append_then_decode(dtype, Hq, Hkv, D, ps
     assert torch.equal(kp_a, kp_b) and torch.equal(vp_a, vp_b)
     assert torch.equal(out_a, out_b)
     assert not torch.equal(kp_b, k_pool)  # the rows were written
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_decode_launch_refuses_a_table_on_another_device(which):
+    """A decode step with cos or sin in host memory raises; nothing is launched."""
+    from nanoslg_amd.kv_cache import KVCacheConfig, PagedKVCache
+    m = PagedKVCache(KVCacheConfig(num_layers=1, num_kv_heads=2, num_qo_heads=8, head_dim=64, max_pages=16, page_size=16,
+                                   dtype=torch.float16, device=DEV, backend="paged"))
+    m.allocate_sequence("a")
+    ctx = m.begin_forward(["a"], [1])
+    q, kv = (torch.zeros(1, 1, h, 64, dtype=torch.float16, device=DEV) for h in (8, 2))
+    tables = [torch.zeros(32, 64, device=DEV) for _ in range(2)]
+    tables[which] = tables[which].cpu()
+    with pytest.raises(ValueError):
+        ctx.attend_rope(0, q, kv, kv, *tables, 8, 2)
