@@ -845,7 +845,7 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
   if (k_new && dtype != NSLG_F16 && dtype != NSLG_BF16)
     return fail(NSLG_EUNSUPPORTED, "paged_prefill_append: dtype %d (f16 or bf16 pools)", dtype);
   if (dtype == NSLG_F32) {
-    // fp32 pools: the VALU attention kernel, ragged rows, bottom-right causal
+    // fp32 pools: the fp32 kernels
     if (q_stride < (int64_t)num_qo_heads * head_dim || out_stride < (int64_t)num_qo_heads * head_dim)
       return fail(NSLG_EINVAL, "paged_prefill: row stride smaller than Hq*D");
     AttnF32Args a;

@@ -273,8 +273,7 @@ def test_missing_library_fails_loudly(tmp_path, monkeypatch):
 
 def test_attention_kernel_rejects_rows_not_16_byte_aligned():
     """Prefill on a padded grid takes only row strides of whole 16-byte units for q and
-    out, on the MFMA kernel (16-bit pools, here at head_dim 256) and on the VALU kernel
-    (fp32 pools) alike: their vector accesses and the pad-row zeroing store 16 bytes at
+    out, in 16-bit pools (here at head_dim 256) and fp32 ones alike: their vector accesses and the pad-row zeroing store 16 bytes at
     a time."""
     from nanoslg_amd import _lib
     lib = _lib.load()

@@ -153,7 +153,7 @@ def test_prefill_attend_takes_strided_kv_rows(monkeypatch):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_head_dim_256_prefill_then_decode(dtype):
     """A 16-bit cache at head_dim 256: a ragged prefill and a chunk over cached
-    context (the VALU attention kernel), then decode steps (the MFMA decode), against
+    context, then decode steps, against
     the oracle: outputs within the tolerance, pad rows zero, pool bytes equal."""
     _log(f"cache: head_dim 256 {dtype}")
     from nanoslg_amd import kv_cache as KC

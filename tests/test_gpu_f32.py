@@ -20,6 +20,7 @@ DEV = "cuda:0"
     ([70, 2000, 0, 33], 32, 8, 64, 48),
     ([31, 900], 12, 2, 256, 16),
     ([700] * 40, 8, 8, 128, 700),                      # whole slots, one run each
+    ([4000, 3100], 32, 8, 128, 16),                    # 32 runs: the merge in four parts
 ])
 def test_f32_decode_edges(lens, Hq, Hkv, D, ps):
     out, ref = _decode_case(lens, Hq, Hkv, D, ps, torch.float32, seed=800 + D + ps)
@@ -33,10 +34,25 @@ def test_f32_decode_edges(lens, Hq, Hkv, D, ps):
     ([1200, 520], [40, 7], 8, 8, 128, 16),                 # runs of keys, merged
     ([700], [300], 16, 1, 64, 1),                          # G = 16, one-token pages
     ([90, 600], [90, 33], 16, 4, 256, 48),
-    ([530] * 24, [40] * 24, 32, 8, 128, 16),               # more workgroups than take two key groups
+    ([530] * 24, [40] * 24, 32, 8, 128, 16),               # two key groups a row tile
+    ([40], [10], 32, 8, 128, 16),                          # too few workgroups for two
+    ([70], [5], 12, 4, 64, 16),
+    ([33, 100], [2, 9], 16, 4, 256, 16),
 ])
 def test_f32_prefill_edges(lens, news, Hq, Hkv, D, ps):
     out, ref = _prefill_case(lens, news, Hq, Hkv, D, ps, torch.float32, seed=820 + D + ps)
+    torch.testing.assert_close(out, ref, **F32_TOL)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_f32_prefill_of_many_workgroups(D):
+    """A ragged batch of more workgroups than take two key groups a row tile, in one run:
+    the kernel of every large fp32 prompt batch."""
+    news = [60 + (7 * b) % 31 for b in range(48)]
+    lens = [n + (5 * b) % 40 for b, n in enumerate(news)]
+    out, ref = _prefill_case(lens, news, 32, 8, D, 16, torch.float32, seed=840 + D)
+    assert (-(-sum(news) * 4 // 64) + len(news)) * 8 > 2048  # launch_f32's limit (D = 64; 1024 otherwise)
     torch.testing.assert_close(out, ref, **F32_TOL)
 
 

@@ -273,8 +273,9 @@ def test_prefill_page_sizes(ps):
 
 
 def test_prefill_long_chunk_and_page_window():
-    """A 512-token chunk over 3584 cached tokens, and a sequence whose page ids span
-    more than one 2048-entry window (page size 1)."""
+    """A 512-token chunk over 3584 cached tokens, and a sequence of more page ids than one
+    2048-entry window (page size 1; its keys are cut into runs, so that no workgroup reloads
+    its window here: test_gpu_prefill_split's page-window test does)."""
     _log("prefill long + window")
     out, ref = _prefill_case([4096, 2500], [512, 300], 32, 8, 128, 16, torch.float16, seed=50)
     torch.testing.assert_close(out, ref, atol=ATOL, rtol=RTOL)
@@ -282,15 +283,16 @@ def test_prefill_long_chunk_and_page_window():
     torch.testing.assert_close(out, ref, atol=ATOL, rtol=RTOL)
 
 
-def test_prefill_row_tile_orders():
-    """Near-uniform batches run their row tiles longest first (rounds sized by the
-    host's max_q); a max_q below a sequence's new tokens, or a ragged batch, takes the
-    packed order. Same results either way."""
-    _log("prefill tile orders")
-    lens, news = [1500, 1400, 1300, 1200], [512, 512, 500, 480]
-    # exact: rounds; understated: the kernel finds a sequence with more tiles than the
-    # rounds cover and packs; far overstated: too many empty slots, packed by the host
-    for max_q in (None, 1, 4096):
+@pytest.mark.parametrize("lens,news", [
+    ([1500, 1400, 1300, 1200], [512, 512, 500, 480]),  # one run whatever max_q says
+    ([3000, 2000], [100, 20]),  # 10 runs; 16 with max_q = 60, which makes a uniform batch of it
+    ([3000, 2000], [64, 64]),   # 16 runs as a uniform batch, 10 with any other max_q
+])
+def test_prefill_max_q_only_sizes_the_runs(lens, news):
+    """max_q sizes the runs that the keys of a call of few row tiles are cut into: one that
+    is exact, too small or too large (0 among them) gives the oracle's result."""
+    _log(f"prefill max_q {news}")
+    for max_q in (None, 60, 0, 1, 4096):
         out, ref = _prefill_case(lens, news, 32, 8, 128, 16, torch.float16, seed=53, max_q=max_q)
         torch.testing.assert_close(out, ref, atol=ATOL, rtol=RTOL)
 
@@ -299,8 +301,8 @@ def test_prefill_row_tile_orders():
 def test_prefill_head_dim_256_chunk_over_cached_context(dtype):
     """16-bit pools at head_dim 256 (the MFMA kernel's shape for it: one 16-row column
     block per wave, 64-key tiles, 128 rows per workgroup): chunks over cached context,
-    GQA 4, 1 and 8, a 512-token chunk over 3584 cached tokens, page sizes 16 and 1 (a
-    sequence whose page ids span more than one 2048-entry window), against the oracle."""
+    GQA 4, 1 and 8, a 512-token chunk over 3584 cached tokens, page sizes 16 and 1, against
+    the oracle."""
     _log(f"prefill D=256 {dtype}")
     out, ref = _prefill_case([300, 1000, 64, 17], [64, 200, 64, 3], 32, 8, 256, 16, dtype, seed=61)
     torch.testing.assert_close(out, ref, atol=ATOL, rtol=RTOL)
@@ -389,7 +391,7 @@ def test_f32_groups_and_page_sizes(Hq, Hkv, ps):
 @pytest.mark.parametrize("lens", [[32768], [9000, 3000, 1, 0], [20000] * 8])
 def test_f32_decode_split_over_keys(lens):
     """Long fp32 decodes are split over keys (partials in the workspace, then an fp32
-    merge): 64, 7 and 8 splits here."""
+    merge): 64, 16 and 8 splits here."""
     _log(f"f32 decode splits lens={lens[:4]}")
     out, ref = _decode_case(lens, 32, 8, 128, 16, torch.float32, seed=len(lens) + lens[0] % 97)
     torch.testing.assert_close(out, ref, **F32_TOL)

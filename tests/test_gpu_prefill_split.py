@@ -1,7 +1,7 @@
 """Prefill calls of few row tiles, whose keys are cut into runs and merged: against the
 oracle's fp32 attention within the attention tolerance, and the forward's K/V write of a
-cut call bit-identical to nslg_append_kv. Keys at the edges of key tiles, runs and page-id
-windows; sequences shorter than a run, without new tokens, and of one new token; padded
+cut call bit-identical to nslg_append_kv. Keys at the edges of key tiles, runs and (in one
+workgroup, cut or not) page-id windows; sequences shorter than a run, without new tokens, and of one new token; padded
 grids; every head dim, GQA group 1, 4 and 16."""
 import numpy as np
 import pytest
@@ -14,7 +14,7 @@ DEV = "cuda:0"
 CASES = [  # lens, new tokens, Hq, Hkv, D, page size
     ([768], [1], 32, 8, 128, 16),               # the shortest sequence that is cut
     ([769], [17], 32, 8, 128, 16),              # a last run of one key
-    ([4096 + 31], [31], 8, 8, 128, 1),          # G = 1, 32 runs across two page-id windows
+    ([4096 + 31], [31], 8, 8, 128, 1),          # G = 1, 32 runs, one-token pages
     ([6000, 300, 900], [33, 0, 5], 32, 8, 128, 16),
     ([1600, 1500], [150, 70], 16, 1, 128, 48),  # G = 16
     ([2100], [300], 32, 8, 64, 16),
@@ -184,3 +184,51 @@ def test_a_callers_workspace_is_used():
     assert torch.cuda.max_memory_allocated() - base <= o2.numel() * 2 + 512
     assert torch.equal(o2, want) and torch.equal(ws.buf, before)
     assert torch.equal(K.paged_decode(dq, k, v, *plan, L // ps, workspace=ws, layout=-101), step)
+
+
+def _room_for(runs, rows, D):
+    """Scratch bytes that hold this many runs of a call of `rows` (token, query head) rows."""
+    up = lambda x: -(-x // 256) * 256  # noqa: E731
+    return 256 + up(rows * 4) + up(rows * runs * 8) + rows * runs * D * 4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("runs,L", [(1, 2070), (2, 4380), (1, 4500)])
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 128), (torch.bfloat16, 64), (torch.bfloat16, 256)])
+def test_a_workgroup_reloads_its_page_window(dtype, D, runs, L, monkeypatch):
+    """Keys of one workgroup past its 2048 page ids (one-token pages): attention against the
+    oracle, and the fused write of new tokens on both sides of the window's end (key 2048 of
+    an uncut call; 4352 and, at D = 256, 4160 in the second of two runs, which begins at
+    2304 and 2112) bit-identical to append_kv."""
+    from nanoslg_amd import kernels as K
+    if runs == 2 and D == 256:
+        L = 4170
+    Hq, Hkv, n, orig = 8, 2, 60, K._prefill_workspace
+    rows = n * Hq
+    room = []
+
+    def cut(*a):
+        if runs == 1:
+            return None, None, 0
+        ws, ptr, nbytes = orig(*a)
+        room.append(ws)
+        assert nbytes >= _room_for(runs, rows, D)
+        return ws, ptr, _room_for(runs, rows, D)
+
+    monkeypatch.setattr(K, "_prefill_workspace", cut)
+    out, ref = _prefill_case([L], [n], Hq, Hkv, D, 1, dtype, seed=L + D)
+    torch.testing.assert_close(out, ref, atol=ATOL, rtol=RTOL)
+    g = torch.Generator().manual_seed(L)
+    ids = torch.randperm(L, generator=g).int()
+    q, k, v = (torch.randn(n, h, D, generator=g).to(dtype).to(DEV) for h in (Hq, Hkv, Hkv))
+    k1, v1 = (torch.randn(L + 3, 1, Hkv, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+    k2, v2 = k1.clone(), v1.clone()
+    i32 = lambda *a: torch.tensor(a, dtype=torch.int32, device=DEV)  # noqa: E731
+    plan = (i32(0, L), ids.to(DEV), i32(1))
+    o1 = K.paged_prefill_append(q, i32(0, n), n, n, k, v, k1, v1, *plan)
+    if runs > 1:
+        assert (room[-1][:rows * 4].view(torch.int32) == runs).all()  # the runs of each row
+    K.append_kv(k, v, ids[L - n:].to(DEV), k2, v2)
+    o2 = K.paged_prefill(q, i32(0, n), n, n, k2, v2, *plan)
+    torch.cuda.synchronize()
+    assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(o1, o2)
