@@ -1823,7 +1823,7 @@ class ContiguousCacheContext(CacheContext):
         pos, q_rows, qo = _ragged_layout(self.start_positions, self.new_token_counts, self.input_offsets, iw)
         self._max_q = max(self.new_token_counts) if B else 0
         self._uniform_rows = int(qo[-1]) == B * iw
-        self._decode_launch = None
+        self._decode_launch = None  # (heads and pools, launcher)
         self._plan = _ForwardPlan(cache.device, B, iw, slot.reshape(-1), pos, indptr, indices, lpl, qo,
                                   q_rows, np.zeros(0, np.int32), np.zeros(0, np.int32))
 
@@ -1835,10 +1835,12 @@ class ContiguousCacheContext(CacheContext):
 
     def attend(self, layer_idx, q, k_new, v_new, n_heads, n_kv_heads):
         cache, plan = self.cache, self._plan
-        if self._in_one_launch(layer_idx, q, k_new, v_new):
-            return self._decode(q)(self._layer(layer_idx), q, k_new, v_new)
-        k_layer, v_layer = cache.paged_view(layer_idx)
         B, S = q.shape[0], q.shape[1]
+        if self._in_one_launch(S, layer_idx, q, k_new, v_new):
+            launch = self._decode(q)
+            if launch is not None:
+                return launch(self._layer(layer_idx), q, k_new, v_new)
+        k_layer, v_layer = cache.paged_view(layer_idx)
         if not (self._is_decode and S == 1):
             # the write and the attention in one launch (a sequence's slot is its one page)
             uniform = self._uniform_rows and S == self._iw
@@ -1861,11 +1863,12 @@ class ContiguousCacheContext(CacheContext):
         cache, plan = self.cache, self._plan
         if self.max_kv_len > cos.shape[0]:
             raise IndexError(f"position {self.max_kv_len - 1} is outside the rope tables ({cos.shape[0]} rows)")
-        if (self._in_one_launch(layer_idx, q, k_new, v_new)
-                and cos.get_device() == sin.get_device() == q.get_device()):
-            return self._decode(q)(self._layer(layer_idx), q, k_new, v_new, rope=(cos, sin, plan.pos_for(1)))
-        k_layer, v_layer = cache.paged_view(layer_idx)
         S = q.shape[1]
+        if self._in_one_launch(S, layer_idx, q, k_new, v_new) and self._rows_to_rotate(q, k_new, v_new):
+            launch = self._decode(q)
+            if launch is not None:
+                return launch(self._layer(layer_idx), q, k_new, v_new, rope=(cos, sin, plan.pos_for(S)))
+        k_layer, v_layer = cache.paged_view(layer_idx)
         q_rot = cache.kernels.rope_append(q, k_new, v_new, plan.pos_for(S), plan.slots_for(S), cos, sin,
                                           k_layer, v_layer)
         return self._attend_written(q_rot, k_layer, v_layer)
@@ -1874,50 +1877,43 @@ class ContiguousCacheContext(CacheContext):
         """A layer index as the pool tensors take it (negative ones from the end)."""
         return layer_idx if layer_idx >= 0 else layer_idx + self.cache.cfg.num_layers
 
-    def _in_one_launch(self, layer_idx, q, k_new, v_new):
-        """A decode step whose rows the decode launch writes itself: one row a sequence, of
-        the pool's dtype and device, q [B, 1, Hq, D] and k_new / v_new [B, 1, Hkv, D] at row
-        strides that do not overlap, q 16-byte aligned. A padded step's row and all other
-        forms take the separate calls, which serve or refuse each as they always did."""
-        if not (self._is_decode and self._iw == 1 and type(layer_idx) is int):
-            return False
-        pool, B = self.cache.k, self.batch_size
-        Hkv, D = pool.shape[3], pool.shape[4]
-        dt, dev = pool.dtype, pool.get_device()
-        if not (q.dtype == k_new.dtype == v_new.dtype == dt
-                and q.get_device() == k_new.get_device() == v_new.get_device() == dev):
-            return False
-        qs, row = q.shape, (B, 1, Hkv, D)
-        if (len(qs) != 4 or qs[0] != B or qs[1] != 1 or qs[3] != D or qs[2] % Hkv or k_new.shape != row
-                or v_new.shape != row):
-            return False
-        st, sk, sv = q.stride(), k_new.stride(), v_new.stride()
-        return (st[3] == sk[3] == sv[3] == 1 and st[2] == sk[2] == sv[2] == D and st[0] >= qs[2] * D
-                and sk[0] >= Hkv * D and sv[0] >= Hkv * D
-                and not (q.data_ptr() | st[0] * q.element_size()) & 15)
+    def _in_one_launch(self, S, layer_idx, q, k_new, v_new):
+        """A decode step whose rows the decode launch writes itself (a padded step's row,
+        tensors of another type and layers not given as an int take the separate calls)."""
+        return (self._is_decode and S == 1 and self._iw == 1 and type(layer_idx) is int
+                and q.dtype == k_new.dtype == v_new.dtype == self.cache.cfg.dtype)
+
+    @staticmethod
+    def _rows_to_rotate(q, k_new, v_new):
+        """Rows that the decode launch rotates itself. nslg_rope_append, which writes rotated
+        q into rows of its own, also takes a single head or a single row at any stride."""
+        st = q.stride()
+        return (len(st) == 4 and st[2] == q.shape[3]
+                and (q.shape[0] > 1 or (st[0] >= q.shape[2] * st[2]
+                                        and not (st[0] | k_new.stride(0) | v_new.stride(0)) & 7)))
 
     def _decode(self, q):
         """The forward's decode launcher (kernels.DecodeLaunch) over the slots, each a page
         of max_seq_len tokens. A launcher belongs to one forward and is bound once, so
-        forwards of one cache can be attended in any order, from several threads too;
-        calls with other heads or after the pools moved get a new one."""
+        forwards of one cache can be attended in any order, from several threads too; a
+        call with other heads, or after the pools moved, gets a new one. None where q's
+        heads are no multiple of the cache's."""
         cache, plan = self.cache, self._plan
-        launch = self._decode_launch
-        if launch is None or not self._serves(launch, q):
+        of = (q.shape[2], cache.k.data_ptr(), cache.v.data_ptr())
+        got = self._decode_launch
+        if got is None or got[0] != of:
+            if of[0] % cache.cfg.num_kv_heads:
+                return None
             prev, kern = cache._launcher, cache.kernels
             args = (plan.slot, plan.indptr, plan.indices, plan.lpl, plan.total_pages)
-            if prev is not None and hasattr(prev, "bound_to") and prev.B == plan.batch and self._serves(prev, q):
+            if (prev is not None and hasattr(prev, "bound_to") and prev.B == plan.batch
+                    and (prev.Hq, prev.kp0, prev.vp0) == of):
                 launch = prev.bound_to(*args)
             else:
                 launch = kern.DecodeLaunch(cache.k, cache.v, *args, q.shape[2], workspace=cache.workspace)
-            self._decode_launch = cache._launcher = launch
-        return launch
-
-    def _serves(self, launch, q):
-        """Whether a launcher made for these pools and heads is one for q's and the cache's."""
-        cache = self.cache
-        return not hasattr(launch, "bound_to") or (
-            launch.Hq == q.shape[2] and launch.kp0 == cache.k.data_ptr() and launch.vp0 == cache.v.data_ptr())
+            cache._launcher = launch
+            self._decode_launch = got = (of, launch)
+        return got[1]
 
     def _attend_written(self, q, k_layer, v_layer):
         """Attention of the forward's rows over the slots (K/V already written)."""

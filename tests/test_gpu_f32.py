@@ -213,7 +213,8 @@ def test_contiguous_forwards_attended_in_between(monkeypatch):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
-FORMS = ["heads", "shared_kv", "flat_kv", "heads_apart", "one_head", "cpu_sin", "cpu_q", "f64_k"]
+FORMS = ["heads", "heads_no_multiple", "shared_kv", "flat_kv", "heads_apart", "one_head", "one_row", "cpu_sin", "cpu_q",
+         "f64_k"]
 
 
 @pytest.mark.gpu
@@ -222,27 +223,33 @@ FORMS = ["heads", "shared_kv", "flat_kv", "heads_apart", "one_head", "cpu_sin", 
 def test_contiguous_decode_takes_the_forms_of_the_separate_calls(form, rope):
     """A decode step of the contiguous cache serves what append_kv (rope_append) and
     paged_decode serve, with their result, and refuses with their error what they refuse:
-    other query heads in one forward, one K row for the whole batch, rows of other ranks,
-    heads apart in memory, tensors of another device or dtype."""
+    other query heads in one forward, heads that are no multiple, one K row for the whole
+    batch, rows of other ranks, heads apart in memory, one head or row at any stride,
+    tensors of another device or dtype."""
     from nanoslg_amd import kernels as K
     from nanoslg_amd.kv_cache import ContiguousKVCache, KVCacheConfig
-    Hq, Hkv, D, B = (1, 1, 64, 2) if form == "one_head" else (8, 2, 64, 2)
+    Hq, Hkv, D, B = (1, 1, 64, 2) if form == "one_head" else (8, 2, 64, 1 if form == "one_row" else 2)
     m = ContiguousKVCache(KVCacheConfig(num_layers=1, num_kv_heads=Hkv, num_qo_heads=Hq, head_dim=D, max_batch_size=B,
                                         max_seq_len=80, dtype=torch.float16, device=torch.device(DEV),
                                         backend="contiguous"))
     g = torch.Generator().manual_seed(6)
     rnd = lambda *s: torch.randn(*s, generator=g).half().to(DEV)  # noqa: E731
-    for s in "ab":
+    ids = ["a", "b"][:B]
+    for s in ids:
         m.allocate_sequence(s)
-    ctx = m.begin_forward(["a", "b"], [40, 3])
+    ctx = m.begin_forward(ids, [40, 3][:B])
     ctx.attend(0, rnd(B, 40, Hq, D), rnd(B, 40, Hkv, D), rnd(B, 40, Hkv, D), Hq, Hkv)
     m.end_forward(ctx)
-    ctx = m.begin_forward(["a", "b"], [1, 1])
+    ctx = m.begin_forward(ids, [1] * B)
     cos, sin = (torch.randn(80, D, generator=g).to(DEV) for _ in range(2))
     q, k, v = rnd(B, 1, Hq, D), rnd(B, 1, Hkv, D), rnd(B, 1, Hkv, D)
     if form == "heads":
         (ctx.attend_rope(0, q, k, v, cos, sin, Hq, Hkv) if rope else ctx.attend(0, q, k, v, Hq, Hkv))
         q = rnd(B, 1, 2 * Hq, D)
+    elif form == "heads_no_multiple":
+        q = rnd(B, 1, 5, D)
+    elif form == "one_row":  # a single row: its stride says nothing
+        q, k, v = (x.as_strided(x.shape, (3, D, D, 1)) for x in (q, k, v))
     elif form == "shared_kv":
         k, v = k[:1].expand(B, 1, Hkv, D), v[:1].expand(B, 1, Hkv, D)
     elif form == "flat_kv":
