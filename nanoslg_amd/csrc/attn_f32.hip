@@ -165,6 +165,7 @@ __global__ void __launch_bounds__(64 * kWavesD) decode_f32_kernel(AttnF32Args p)
   const int piece = ((L + p.splits - 1) / p.splits + kRunD - 1) / kRunD * kRunD;
   const int kv_begin = min(L, split * piece);
   const int kv_end = min(L, kv_begin + piece);
+  if (p.ws_tag && blockIdx.x == 0 && split == 0 && threadIdx.x == 0) *p.ws_tag = 0;
   const int64_t rows = (int64_t)p.batch * p.num_qo_heads;
   const int64_t prow0 = (int64_t)b * p.num_qo_heads + h * G;
   if (kv_begin >= kv_end && p.splits > 1) {  // uniform: no key, no share in the merge
@@ -328,6 +329,7 @@ __global__ void __launch_bounds__(256 * kGroups) prefill_f32_kernel(AttnF32Args 
   if (p.q_rows)
     zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, p.batch, p.out, p.out_stride * 4, p.num_qo_heads * D * 4,
                   blockIdx.x * (kThreads / 64) + (tid >> 6), gridDim.x * (kThreads / 64));
+  if (p.ws_tag && blockIdx.x == 0 && tid == 0) *p.ws_tag = 0;
   const int runs = p.num_kv_heads * p.splits;
   const int run = blockIdx.x % runs;
   const int split = run / p.num_kv_heads, h = run - split * p.num_kv_heads;  // a head's runs on one XCD
@@ -637,7 +639,7 @@ int attention_f32_prefill_splits(int64_t total_q, int32_t num_qo_heads, size_t w
 
 size_t attention_f32_workspace(int64_t total_q, int32_t num_qo_heads, int32_t head_dim, int splits) {
   if (splits <= 1) return 256;
-  return (size_t)total_q * num_qo_heads * splits * (head_dim + 2) * sizeof(float) + 256;
+  return (size_t)total_q * num_qo_heads * splits * (head_dim + 2) * sizeof(float) + 512;
 }
 
 int attention_f32(const AttnF32Args& a, int32_t head_dim, hipStream_t s) {
@@ -657,8 +659,9 @@ int attention_f32(const AttnF32Args& a, int32_t head_dim, hipStream_t s) {
   if (a.q_rows && (!a.qo_indptr || a.grid_width < 1))
     return fail(NSLG_EINVAL, "attention_f32: a padded grid needs ragged rows and a width");
   AttnF32Args p = a;
-  if (a.splits > 1) {  // part_o [splits, rows, D], part_ml [splits, rows, 2]
-    p.part_o = (float*)(((uintptr_t)a.workspace + 255) / 256 * 256);
+  if (a.splits > 1) {  // the first word, part_o [splits, rows, D], part_ml [splits, rows, 2]
+    p.ws_tag = (uint64_t*)(((uintptr_t)a.workspace + 255) / 256 * 256);
+    p.part_o = (float*)(p.ws_tag + 32);
     p.part_ml = p.part_o + a.total_q * a.num_qo_heads * a.splits * head_dim;
   }
   dim3 grid;

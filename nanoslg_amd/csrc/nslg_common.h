@@ -322,6 +322,7 @@ struct AttnF32Args {
   int32_t splits;              // runs of keys per row tile (1: no partials)
   void* workspace = nullptr;   // splits > 1: attention_f32_workspace bytes
   // set by attention_f32
+  uint64_t* ws_tag = nullptr;  // splits > 1: the workspace's first word, set to 0 (see ws_tag in paged_prefill.hip)
   float* part_o = nullptr;     // [splits, total_q, Hq, D] partial outputs
   float* part_ml = nullptr;    // [splits, total_q, Hq, 2] running max and sum
 };

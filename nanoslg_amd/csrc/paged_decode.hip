@@ -65,7 +65,10 @@ struct DecodeParams {
   // Layout of the call's chunks, kept in the workspace for the other layers of a
   // forward (same batch and plan): layout_mode 0: found from the lengths; > 0: found,
   // and recorded under layout_tag; < 0: read from the record when *layout_tag_ptr is
-  // layout_tag, found otherwise. Two int4 per chunk (see the kernel).
+  // layout_tag, found otherwise. Two int4 per chunk (see the kernel). The tag is the
+  // workspace's first word, which every call that does not read its own record sets (0:
+  // none), as every other kernel that puts partials into a workspace does: no call that
+  // may have written over the record leaves its tag.
   int32_t layout_mode;
   int64_t total_pages;  // entries of indices (kv_indptr[batch])
   uint64_t layout_tag;
@@ -446,7 +449,7 @@ paged_decode_kernel(DecodeParams p, GroupArgs<kGrouped> ga) {
   if (!mapped) {
     g = -1;
     merged = false;
-    if (record && chunk == 0) *p.layout_tag_ptr = p.layout_tag;
+    if (chunk == 0 && blockIdx.y == 0 && threadIdx.x == 0) *p.layout_tag_ptr = p.layout_mode > 0 ? p.layout_tag : 0;
     int units = p.batch;
     if constexpr (kGrouped) units += ga.num_groups;
     const LaneLens<kGrouped> lens(p, ga, units);
@@ -1101,15 +1104,16 @@ int launch_decode(const DecodeParams& p, const MergeParams& mp, const GroupArgs<
 
 inline size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Workspace: partials [max_chunks, slot_members, Hq, D] and [..., 2] fp32, then each
-// sequence's chunk range, then each group prefix's chunk range (int32 pairs), then
-// the recorded chunk layout (a 16-byte tag, then two int4 per chunk), each region
-// rounded up to 256 bytes.
+// Workspace: the recorded chunk layout (a 16-byte tag, then two int4 per chunk), partials
+// [max_chunks, slot_members, Hq, D] and [..., 2] fp32, then each sequence's chunk range,
+// then each group prefix's chunk range (int32 pairs), each region rounded up to 256 bytes.
+inline size_t layout_bytes(const DecodeShape& sh) { return round256(16 + (size_t)sh.max_chunks * 32); }
+
 size_t workspace_bytes_for(const DecodeShape& sh, int32_t batch, int32_t num_qo_heads, int32_t head_dim,
                            int32_t slot_members, int32_t num_groups) {
-  return (size_t)(sh.max_chunks * slot_members * num_qo_heads * (head_dim + 2) * (int64_t)sizeof(float)) +
-         round256((size_t)batch * 8) + (num_groups > 0 ? round256((size_t)num_groups * 8) : 0) +
-         round256(16 + (size_t)sh.max_chunks * 32);
+  return layout_bytes(sh) +
+         (size_t)(sh.max_chunks * slot_members * num_qo_heads * (head_dim + 2) * (int64_t)sizeof(float)) +
+         round256((size_t)batch * 8) + (num_groups > 0 ? round256((size_t)num_groups * 8) : 0);
 }
 
 bool shape_ok(int32_t batch, int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim, int64_t total_pages,
@@ -1291,16 +1295,15 @@ int decode_impl(const void* q, int64_t q_stride, const void* k_pool, const void*
   p.rope_stride = nr.table_stride;
   p.rope_rows = nr.table_rows;
   char* ws = (char*)workspace;
-  p.part_o = (float*)ws;
-  p.part_ml = p.part_o + mc * slot_members * num_qo_heads * head_dim;
-  char* meta = ws + (size_t)(mc * slot_members * num_qo_heads * (head_dim + 2) * (int64_t)sizeof(float));
-  p.meta = reinterpret_cast<int2*>(meta);
-  if constexpr (kGrouped) ga.group_meta = reinterpret_cast<int2*>(meta + round256((size_t)batch * 8));
-  char* lay = meta + round256((size_t)batch * 8) + (num_groups > 0 ? round256((size_t)num_groups * 8) : 0);
   p.layout_mode = layout > 0 ? 1 : (layout < 0 ? -1 : 0);
   p.layout_tag = (uint64_t)(layout > 0 ? layout : -layout);
-  p.layout_tag_ptr = reinterpret_cast<uint64_t*>(lay);
-  p.layout_map = reinterpret_cast<int4*>(lay + 16);
+  p.layout_tag_ptr = reinterpret_cast<uint64_t*>(ws);
+  p.layout_map = reinterpret_cast<int4*>(ws + 16);
+  p.part_o = (float*)(ws + layout_bytes(sh));
+  p.part_ml = p.part_o + mc * slot_members * num_qo_heads * head_dim;
+  char* meta = reinterpret_cast<char*>(p.part_ml + mc * slot_members * num_qo_heads * 2);
+  p.meta = reinterpret_cast<int2*>(meta);
+  if constexpr (kGrouped) ga.group_meta = reinterpret_cast<int2*>(meta + round256((size_t)batch * 8));
   p.total_pages = total_pages;
 
   MergeParams mp;

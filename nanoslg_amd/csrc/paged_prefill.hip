@@ -108,6 +108,9 @@ struct PrefillParams {
   // part_count holds the runs of each (token, head): 1 for a row already in `out`.
   int32_t splits;
   int64_t total_q;
+  // the workspace's first word, set to 0: a decode call's chunk layout recorded in the same
+  // memory (its tag there) is not to be read after the partials went over it
+  uint64_t* ws_tag;
   float* part_o;        // [splits, total_q, Hq, D]
   float2* part_ml;      // [splits, total_q, Hq]: running max (log2 units) and row sum
   int32_t* part_count;  // [total_q, Hq]
@@ -172,6 +175,7 @@ __global__ void __launch_bounds__(64 * PrefillTile<D>::kWaves) paged_prefill_ker
   if (p.q_rows)
     zero_pad_rows(p.qo_indptr, p.q_rows, p.grid_width, p.batch, p.out, p.out_stride * 2, p.num_qo_heads * D * 2,
                   w * kWaves + wave, p.num_work * kWaves);
+  if (kSplit && w == 0 && tid == 0) *p.ws_tag = 0;
   const int runs = kSplit ? p.num_kv_heads * p.splits : p.num_kv_heads;
   const int run = w % runs;
   const int h = kSplit ? run % p.num_kv_heads : run;
@@ -792,11 +796,12 @@ int prefill_splits(int64_t total_q, int32_t batch, int32_t max_q, int group, int
   return (int)(s < 1 ? 1 : (s > kMaxSplits ? kMaxSplits : s));
 }
 
-// Partials of `splits` runs of total_q x Hq rows: part_count, part_ml, part_o.
+// Workspace of `splits` runs of total_q x Hq rows: the first word, part_count, part_ml,
+// part_o, and what rounding its address up to 256 bytes may take.
 size_t split_bytes(int64_t rows, int splits, int head_dim) {
   const size_t count = ((size_t)rows * 4 + 255) / 256 * 256;
   const size_t ml = ((size_t)rows * splits * 8 + 255) / 256 * 256;
-  return 256 + count + ml + (size_t)rows * splits * head_dim * 4;
+  return 512 + count + ml + (size_t)rows * splits * head_dim * 4;
 }
 
 }  // namespace
@@ -924,6 +929,7 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
   if (tiles * num_kv_heads * kMaxSplits > 0x7fffffff) return fail(NSLG_EUNSUPPORTED, "paged_prefill: too many rows");
   p.total_q = total_q;
   p.splits = 1;
+  p.ws_tag = nullptr;
   p.part_o = nullptr;
   p.part_ml = nullptr;
   p.part_count = nullptr;
@@ -934,6 +940,8 @@ int prefill_impl(const void* q, int64_t q_stride, const int32_t* qo_indptr, cons
     if (s > 1) {
       char* ws = (char*)(((uintptr_t)workspace + 255) / 256 * 256);  // (split_bytes has room for this)
       p.splits = s;
+      p.ws_tag = (uint64_t*)ws;
+      ws += 256;
       p.part_count = (int32_t*)ws;
       ws += ((size_t)rows * 4 + 255) / 256 * 256;
       p.part_ml = (float2*)ws;

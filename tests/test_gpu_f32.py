@@ -286,3 +286,53 @@ def test_contiguous_decode_takes_the_forms_of_the_separate_calls(form, rope):
     out = call()
     torch.cuda.synchronize()
     assert torch.equal(out, want) and torch.equal(m.k[0], kc) and torch.equal(m.v[0], vc)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("backend", ["contiguous", "paged"])
+@pytest.mark.parametrize("others", [1, 70])
+def test_decode_forwards_of_other_batches_in_between(backend, others):
+    """The layers of a decode forward of 40 sequences with another forward's layer after
+    each: the chunk layout recorded by the first layer is not read once the other forward's
+    call has used the workspace, whatever its size. Outputs and pools as with the forwards
+    one after the other."""
+    from nanoslg_amd.kv_cache import ContiguousKVCache, KVCacheConfig, PagedKVCache
+    L, Hq, Hkv, D, B = 3, 8, 2, 64, 40
+    ids = ["s%d" % i for i in range(B + others)]
+    lens = [100 + 37 * i % 900 for i in range(B)] + [20 + i for i in range(others)]
+    cfg = dict(num_layers=L, num_kv_heads=Hkv, num_qo_heads=Hq, head_dim=D, dtype=torch.float16,
+               device=torch.device(DEV), backend=backend)
+
+    def outputs(in_turn):
+        g = torch.Generator().manual_seed(8)
+        rnd = lambda *s: torch.randn(*s, generator=g).half().to(DEV)  # noqa: E731
+        if backend == "paged":
+            m = PagedKVCache(KVCacheConfig(max_pages=sum(-(-n // 16) + 1 for n in lens) + 2, page_size=16,
+                                           enable_prefix_caching=False, **cfg))
+        else:
+            m = ContiguousKVCache(KVCacheConfig(max_batch_size=len(ids), max_seq_len=1024, **cfg))
+        for s in ids:
+            m.allocate_sequence(s)
+        m.end_forward(m.begin_forward(ids, lens))
+        pool = m if backend == "contiguous" else m.pool
+        pool.k.copy_(rnd(*pool.k.shape))
+        pool.v.copy_(rnd(*pool.v.shape))
+        batches = [ids[:B], ids[B:]]
+        inputs = [[(rnd(len(b), 1, Hq, D), rnd(len(b), 1, Hkv, D), rnd(len(b), 1, Hkv, D)) for _ in range(L)]
+                  for b in batches]
+        out = []
+        if in_turn:
+            forwards = [m.begin_forward(b, [1] * len(b)) for b in batches]
+            for layer in range(L):
+                out += [f.attend(layer, *x[layer], Hq, Hkv) for f, x in zip(forwards, inputs)]
+        else:
+            done = []
+            for b, x in zip(batches, inputs):
+                f = m.begin_forward(b, [1] * len(b))
+                done.append([f.attend(layer, *x[layer], Hq, Hkv) for layer in range(L)])
+            out = [o for pair in zip(*done) for o in pair]
+        torch.cuda.synchronize()
+        return out + [pool.k, pool.v]
+
+    for a, b in zip(outputs(True), outputs(False)):
+        assert torch.equal(a, b)

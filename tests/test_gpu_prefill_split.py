@@ -189,7 +189,7 @@ def test_a_callers_workspace_is_used():
 def _room_for(runs, rows, D):
     """Scratch bytes that hold this many runs of a call of `rows` (token, query head) rows."""
     up = lambda x: -(-x // 256) * 256  # noqa: E731
-    return 256 + up(rows * 4) + up(rows * runs * 8) + rows * runs * D * 4
+    return 512 + up(rows * 4) + up(rows * runs * 8) + rows * runs * D * 4
 
 
 @pytest.mark.gpu
@@ -227,8 +227,36 @@ def test_a_workgroup_reloads_its_page_window(dtype, D, runs, L, monkeypatch):
     plan = (i32(0, L), ids.to(DEV), i32(1))
     o1 = K.paged_prefill_append(q, i32(0, n), n, n, k, v, k1, v1, *plan)
     if runs > 1:
-        assert (room[-1][:rows * 4].view(torch.int32) == runs).all()  # the runs of each row
+        assert (room[-1][256:256 + rows * 4].view(torch.int32) == runs).all()  # the runs of each row
     K.append_kv(k, v, ids[L - n:].to(DEV), k2, v2)
     o2 = K.paged_prefill(q, i32(0, n), n, n, k2, v2, *plan)
     torch.cuda.synchronize()
     assert torch.equal(k1, k2) and torch.equal(v1, v2) and torch.equal(o1, o2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["prefill", "prefill_f32", "decode_f32", "decode"])
+def test_partials_void_a_recorded_chunk_layout(call, monkeypatch):
+    """A workspace that holds a decode call's chunk layout, then another call's partials: the
+    layout's tag is gone, and the decode's next layer cuts its chunks anew."""
+    from nanoslg_amd import kernels as K
+    Hq, Hkv, D, ps, L, n = 8, 2, 128, 16, 4000, 20
+    g = torch.Generator().manual_seed(4)
+    rnd = lambda *s: torch.randn(*s, generator=g).half().to(DEV)  # noqa: E731
+    k, v, q, dq = rnd(L // ps, ps, Hkv, D), rnd(L // ps, ps, Hkv, D), rnd(n, Hq, D), rnd(1, Hq, D)
+    d = lambda *a: torch.tensor(a, dtype=torch.int32, device=DEV)  # noqa: E731
+    plan = (d(0, L // ps), torch.arange(L // ps, dtype=torch.int32, device=DEV), d(ps))
+    ws = K.Workspace(DEV, 64 << 20)
+    tag = lambda: int(ws.buf[:8].view(torch.int64))  # noqa: E731
+    step = K.paged_decode(dq, k, v, *plan, L // ps, workspace=ws, layout=102)
+    assert tag() == 102
+    monkeypatch.setattr(K.Workspace, "get_prefill", K.Workspace.get)  # one memory for both, as in a C program
+    if call.startswith("prefill"):
+        x = [t.float() for t in (q, k, v)] if call.endswith("f32") else [q, k, v]
+        K.paged_prefill(x[0], d(0, n), n, n, x[1], x[2], *plan, workspace=ws)
+    elif call == "decode_f32":
+        K.paged_decode(dq.float(), k.float(), v.float(), *plan, L // ps, workspace=ws)
+    else:
+        K.paged_decode(dq, k, v, *plan, L // ps, workspace=ws)
+    assert tag() == 0
+    assert torch.equal(K.paged_decode(dq, k, v, *plan, L // ps, workspace=ws, layout=-102), step)
