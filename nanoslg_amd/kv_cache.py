@@ -1824,6 +1824,9 @@ class ContiguousCacheContext(CacheContext):
         self._max_q = max(self.new_token_counts) if B else 0
         self._uniform_rows = int(qo[-1]) == B * iw
         self._decode_launch = None  # (heads and pools, launcher)
+        # a decode step whose rows the decode launch writes itself (a padded step's row, tensors
+        # of another type and layers not given as an int take the separate calls)
+        self._one_row, self._dtype = self._is_decode and iw == 1, cfg.dtype
         self._plan = _ForwardPlan(cache.device, B, iw, slot.reshape(-1), pos, indptr, indices, lpl, qo,
                                   q_rows, np.zeros(0, np.int32), np.zeros(0, np.int32))
 
@@ -1836,10 +1839,11 @@ class ContiguousCacheContext(CacheContext):
     def attend(self, layer_idx, q, k_new, v_new, n_heads, n_kv_heads):
         cache, plan = self.cache, self._plan
         B, S = q.shape[0], q.shape[1]
-        if self._in_one_launch(S, layer_idx, q, k_new, v_new):
+        if (self._one_row and S == 1 and type(layer_idx) is int
+                and q.dtype == k_new.dtype == v_new.dtype == self._dtype):
             launch = self._decode(q)
             if launch is not None:
-                return launch(self._layer(layer_idx), q, k_new, v_new)
+                return launch(layer_idx if layer_idx >= 0 else layer_idx + cache.cfg.num_layers, q, k_new, v_new)
         k_layer, v_layer = cache.paged_view(layer_idx)
         if not (self._is_decode and S == 1):
             # the write and the attention in one launch (a sequence's slot is its one page)
@@ -1864,24 +1868,16 @@ class ContiguousCacheContext(CacheContext):
         if self.max_kv_len > cos.shape[0]:
             raise IndexError(f"position {self.max_kv_len - 1} is outside the rope tables ({cos.shape[0]} rows)")
         S = q.shape[1]
-        if self._in_one_launch(S, layer_idx, q, k_new, v_new) and self._rows_to_rotate(q, k_new, v_new):
+        if (self._one_row and S == 1 and type(layer_idx) is int
+                and q.dtype == k_new.dtype == v_new.dtype == self._dtype and self._rows_to_rotate(q, k_new, v_new)):
             launch = self._decode(q)
             if launch is not None:
-                return launch(self._layer(layer_idx), q, k_new, v_new, rope=(cos, sin, plan.pos_for(S)))
+                return launch(layer_idx if layer_idx >= 0 else layer_idx + cache.cfg.num_layers, q, k_new, v_new,
+                              rope=(cos, sin, plan.pos_for(S)))
         k_layer, v_layer = cache.paged_view(layer_idx)
         q_rot = cache.kernels.rope_append(q, k_new, v_new, plan.pos_for(S), plan.slots_for(S), cos, sin,
                                           k_layer, v_layer)
         return self._attend_written(q_rot, k_layer, v_layer)
-
-    def _layer(self, layer_idx):
-        """A layer index as the pool tensors take it (negative ones from the end)."""
-        return layer_idx if layer_idx >= 0 else layer_idx + self.cache.cfg.num_layers
-
-    def _in_one_launch(self, S, layer_idx, q, k_new, v_new):
-        """A decode step whose rows the decode launch writes itself (a padded step's row,
-        tensors of another type and layers not given as an int take the separate calls)."""
-        return (self._is_decode and S == 1 and self._iw == 1 and type(layer_idx) is int
-                and q.dtype == k_new.dtype == v_new.dtype == self.cache.cfg.dtype)
 
     @staticmethod
     def _rows_to_rotate(q, k_new, v_new):
