@@ -131,14 +131,16 @@ int nslg_gather_kv(const void* k_pool, const void* v_pool, int64_t num_pages,
  *   sm_scale          softmax scale (1/sqrt(D) for the reference)
  *   workspace         caller-owned device scratch of at least
  *                     nslg_paged_decode_workspace_size(...) bytes, 256-byte aligned;
- *                     one call at a time per workspace
+ *                     one call at a time per workspace (calls of any kind may take
+ *                     it in turn)
  *   layout            0: the call cuts its sequences into chunks from their lengths
  *                     (every wave reads the lengths and searches the chunk length);
  *                     t > 0: the same, and the chunks' work is recorded in the
  *                     workspace under tag t; -t: a later call of the same forward
  *                     (another layer: same batch, block table, lengths, sizes and
  *                     workspace) reads the record instead, when the workspace still
- *                     holds tag t (else it cuts the chunks itself). Results are
+ *                     holds tag t (its first word, which every call that puts partials
+ *                     into a workspace sets; else it cuts the chunks itself). Results are
  *                     bit-identical in all three modes; a tag must not be reused for
  *                     another forward (a wrong record gives wrong results, though
  *                     every access stays inside the block table and the pool).
@@ -351,7 +353,10 @@ int nslg_paged_decode_grouped_rope_append(
  *   workspace   of nslg_paged_prefill_workspace_size bytes, not shared with a call
  *               that may run at the same time: a call of few row tiles then cuts its
  *               keys into runs and merges them (a second launch). Null or smaller:
- *               fewer runs, or one and no use of the workspace
+ *               fewer runs, or one and no use of the workspace. The merge costs about
+ *               8 us whatever the keys, which only the caller knows on the host: calls
+ *               whose sequences are all short (below about 768 tokens; 1024 at D = 64)
+ *               are faster with null
  * Supported: f16, bf16 with D in {64, 128, 256} (MFMA); f32 with D in {64, 128,
  * 256} (fp32 MFMA, attn_f32.hip); 1 <= Hq/Hkv <= 16.
  */
@@ -381,7 +386,7 @@ int nslg_paged_prefill(const void* q, int64_t q_stride, const int32_t* qo_indptr
  * on and the unpack of its output into the padded grid (kv_cache.py:676-691):
  * the kernel reads and writes the grid rows directly. q_rows: int32[total_q]
  * (device); a row outside the grid is neither read nor written. Other arguments
- * as nslg_paged_prefill (workspace unused).
+ * as nslg_paged_prefill.
  */
 int nslg_paged_prefill_grid(const void* q, int64_t q_stride, const int32_t* qo_indptr,
                             const int32_t* q_rows, int32_t grid_width, int64_t total_q,
@@ -401,7 +406,7 @@ int nslg_paged_prefill_grid(const void* q, int64_t q_stride, const int32_t* qo_i
  * nanoslg/kv_cache.py:661-674, slots of :575-594) together with the prefill run
  * (:657-659), which the reference issues back to back for one forward (:639-659).
  * Same result as nslg_append_kv of the rows followed by nslg_paged_prefill (q_rows
- * null) or nslg_paged_prefill_grid (q_rows set), bit for bit.
+ * null) or nslg_paged_prefill_grid (q_rows set) with as much workspace, bit for bit.
  *
  *   k_new, v_new   rows of Hkv*D elements at element strides k_new_stride,
  *                  v_new_stride (device, the pool's dtype, 16-byte aligned rows),

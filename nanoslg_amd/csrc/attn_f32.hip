@@ -600,8 +600,8 @@ int launch_f32(const AttnF32Args& p, dim3 grid, hipStream_t s) {
     // Two groups of waves on each row tile, half of an LDS tile's keys each, where one group
     // leaves SIMDs idle: fresh prompts of few tiles (4 x 128 tokens 25.5 -> 24.0 us, 4 x
     // 100..512 47.6 -> 42.4; D = 64, 4 x 512, 105 -> 84). Not for calls of many workgroups
-    // (8 x 512 over 512: 542 us, with two groups 646), calls cut into runs (512 from zero
-    // 57.3 and 63.5), nor a few short tiles (16 tokens 10.9 and 12.5).
+    // (8 x 512 over 512: 542 us, with two groups 646), calls cut into runs (512 from zero, in
+    // a call given a workspace, 57.3 and 63.5), nor a few short tiles (16 tokens 10.9 and 12.5).
     if (p.splits == 1 && grid.x > 32 && grid.x <= (D == 64 ? 2048u : 1024u))
       prefill_f32_kernel<D, 2><<<grid, 512, 0, s>>>(p);
     else
